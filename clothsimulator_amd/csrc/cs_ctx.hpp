@@ -116,6 +116,7 @@ struct ClothSys {
     int mesh;
     unsigned asmEpoch = 0;  // incremented by every assembly of the system
     int nn, nslices, totalSlots, maxWidth;
+    int bandwidth = 0;  // largest |column - row| of the static pattern
     // static sliced-ELL pattern
     DBuf sliceOff;  // int[nslices+1] (in slots)
     DBuf sliceW;    // int[nslices]
@@ -248,6 +249,9 @@ struct cs_ctx {
     // PCG
     cs::DBuf pcgPartial, pcgScal, pcgCounter;
     cs::PcgScalars* hScal = nullptr;  // pinned
+    // whole solves in one launch (cs_ppcg.hip): system table, block -> (system, workgroup) map, slots
+    cs::DBuf ppTab, ppMap, ppSlots;
+    bool ppOff = false;  // refused a launch: solve with separate launches
     // batched solve of independent cloths: per-cloth table, block -> cloth map, partials, scalars
     cs::DBuf bTab, bMap, bPart, bScal, bList;
     struct BatchTune {

@@ -216,6 +216,7 @@ static void build_cloth_system(cs_ctx* C, int c, ClothSys& S) {
     S.hRowPtr.assign(M.nn + 1, 0);
     S.hRowLen.assign(M.nn, 0);
     S.hCol.clear();
+    S.bandwidth = 0;
     for (int i = 0; i < M.nn; i++) {
         std::vector<int>& r = adj[i];
         std::sort(r.begin(), r.end());
@@ -224,6 +225,7 @@ static void build_cloth_system(cs_ctx* C, int c, ClothSys& S) {
         S.hRowLen[i] = (int)r.size();
         S.hRowPtr[i + 1] = S.hRowPtr[i] + (int)r.size();
         S.hCol.insert(S.hCol.end(), r.begin(), r.end());
+        if (!r.empty()) S.bandwidth = std::max(S.bandwidth, std::max(i - r.front(), r.back() - i));
     }
     S.nslices = cdiv(M.nn, SLICE);
     S.hSliceOff.assign(S.nslices + 1, 0);

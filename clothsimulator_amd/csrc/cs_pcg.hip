@@ -1001,6 +1001,20 @@ __global__ void __launch_bounds__(BP) k_bpcg_recheck(const BCloth* __restrict__ 
 
 int pcg_solve(cs_ctx* C, int c, float* relres, int* converged) {
     ClothSys& S = C->sys[c];
+    // Block Jacobi (and a cloth too small for the multigrid it asks for) is solved inside one launch
+    // where its matrix fits the chip's registers; timed runs keep the launches they time.
+    int small[16];
+    const bool jacobi = C->P.precond == CS_PRECOND_BLOCK_JACOBI ||
+                        (C->P.precond != CS_PRECOND_LEARNED && amg_levels(C, c, small, 16) <= 1);
+    if (jacobi && !(C->P.flags & CS_FLAG_TIME_KERNELS)) {
+        int it = 0, conv = 0;
+        float rel = 0.0f;
+        if (ppcg_solve(C, {c}, &it, &rel, &conv)) {
+            if (relres) *relres = rel;
+            if (converged) *converged = conv;
+            return it;
+        }
+    }
     hipStream_t s = C->stream;
     const int nn = S.nn;
     const int nb = std::min(PMAX, (cdiv(nn, PB) + 7) & ~7);
@@ -1447,7 +1461,14 @@ void pcg_solve_batched(cs_ctx* C, int* iters, float* relres, int* converged, boo
     else if (tuning) cand = T.trials % kTuneN;
     const auto t0 = std::chrono::steady_clock::now();
     const int chunk = amg ? kTuneChunk[cand] / 4 : kTuneChunk[cand];
-    if (kTuneRows[cand] == 128) solve_batched<128>(C, chunk, iters, relres, converged, amg);
+    // block Jacobi: every cloth's whole solve inside one or two launches where the matrices fit the
+    // chip (no candidate applies there: a cloth's result is that of its own single solve, bit for
+    // bit); timed runs keep the launches they time
+    std::vector<int> every(C->nCloths);
+    for (int c = 0; c < C->nCloths; c++) every[c] = c;
+    const bool onchip = !amg && !(C->P.flags & CS_FLAG_TIME_KERNELS) && ppcg_solve(C, every, iters, relres, converged);
+    if (onchip) {
+    } else if (kTuneRows[cand] == 128) solve_batched<128>(C, chunk, iters, relres, converged, amg);
     else solve_batched<256>(C, chunk, iters, relres, converged, amg);
     if (tuning) {
         const double sec = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();

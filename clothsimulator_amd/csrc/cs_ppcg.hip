@@ -1,0 +1,622 @@
+// cs_ppcg.hip — block-Jacobi PCG of whole systems in one launch, the matrix held in registers.
+//
+// A separately launched iteration (cs_pcg.hip) of a system of 16,641 rows or fewer takes 13-14 us,
+// nearly all of it latency: two kernel boundaries, and in each kernel a chain of dependent loads.
+// The chip's registers hold the matrices of 131,072 rows: here a thread owns one row for the whole
+// solve and keeps its 3x3 blocks (RS of them), its columns as 16-bit offsets, and its r, x, z, d, q
+// in registers.  An iteration then moves only vectors: a thread publishes its z and d and gathers
+// its neighbours'.
+//
+// A system is solved by a group of workgroups, T rows each, that meet twice an iteration: when
+// z and the partials of r.z and r.r are out, and when the partial of d.q is.  The meeting is an
+// all-reduce: each workgroup stores (epoch, value) words to its slots, every workgroup polls all
+// slots of its group, and forms the sums in the order of the separate launches: the solve gives
+// their bits, whatever it shares a launch with (1.0 us for 2 workgroups, 1.4 us for 17, 2.9 us for 256; a
+// cooperative-groups grid barrier took 700 us for 1,536 because every wave wrote its L2 back).
+// No L2 write-back is needed: what others read is stored with agent-scope atomic stores, which
+// write through.  Groups are independent, so one launch solves many systems.
+//
+// The whole solve is in the kernel: start, iterations, the check of the true residual with FP64 row
+// sums and the continuations from it, as pcg_solve's.  The workgroups of a group wait for each
+// other, so they must all be resident: launches are cooperative and no larger than the device
+// holds at once.  One process at a time gets a device's cooperative queue: where the launch is
+// refused, and if a wait (each is bounded in time) runs out, the context solves with separate
+// launches from then on.
+//
+// Measured (solve time per iteration, separate launches -> here): 289 rows 14.1 -> 2.8 us,
+// 1,089 rows 13.5 -> 4.6, 16,641 rows with contacts 13.6 -> 7.9, 32,761 rows 13.9 -> 7.1,
+// 65,536 rows 18.0 -> 9.1, 129,600 rows 21.6 -> 15.3.
+#include <algorithm>
+#include <cfloat>
+#include <cmath>
+#include <cstring>
+
+#include "cs_kernels.hpp"
+#include "cs_math.hpp"
+
+namespace cs {
+
+namespace {
+
+constexpr int RESTARTS = 4;                      // continuations from the true residual, as pcg_solve
+constexpr unsigned long long WAIT_TICKS = 200000000ull;  // 2 s of the 100 MHz wall clock
+
+struct PSys {
+    int nn, nslices, G, contacts;
+    const int *sliceOff, *sliceW, *cols, *cRowPtr, *cCol;
+    const float *vals, *cVal, *Minv, *b, *bc;
+    float* x;
+    float4 *z, *d;      // z: nn, d: two generations of nn
+    uint64_t* slots;    // 2 generations x 2 values x (G * T / BLK) words (epoch << 32 | value), zero at launch
+    PcgScalars* out;
+};
+
+// The pointers in the global address space (cs_math.hpp, G1)
+struct PSysG {
+    int nn, nslices, G, contacts;
+    const G1<int> *sliceOff, *sliceW, *cols, *cRowPtr, *cCol;
+    const G1<float> *vals, *cVal, *Minv, *b, *bc;
+    G1<float>* x;
+    G1<f4n> *z, *d;
+    G1<uint64_t>* slots;
+    PcgScalars* out;
+};
+__device__ __forceinline__ PSysG gview(const PSys& c) {
+    PSysG g;
+    g.nn = c.nn;
+    g.nslices = c.nslices;
+    g.G = c.G;
+    g.contacts = c.contacts;
+    g.sliceOff = g1(c.sliceOff); g.sliceW = g1(c.sliceW); g.cols = g1(c.cols);
+    g.cRowPtr = g1(c.cRowPtr); g.cCol = g1(c.cCol);
+    g.vals = g1(c.vals); g.cVal = g1(c.cVal); g.Minv = g1(c.Minv); g.b = g1(c.b); g.bc = g1(c.bc);
+    g.x = g1(c.x);
+    g.z = (G1<f4n>*)c.z;
+    g.d = (G1<f4n>*)c.d;
+    g.slots = g1(c.slots);
+    g.out = c.out;
+    return g;
+}
+
+__device__ __forceinline__ void put64(G1<uint64_t>* p, uint64_t v) {
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ uint64_t get64(const G1<uint64_t>* p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+// publishes a row's vector for the other workgroups
+__device__ __forceinline__ void put3(G1<f4n>* p, V3f a) {
+    G1<uint64_t>* q = (G1<uint64_t>*)p;
+    put64(q, (uint64_t)__float_as_uint(a.y) << 32 | __float_as_uint(a.x));
+    put64(q + 1, __float_as_uint(a.z));
+}
+
+// Element at a 32-bit byte offset from a uniform base: one scalar base and one offset register
+// per access (systems here stay far below 4 GB).
+template <class V> __device__ __forceinline__ G1<V>& at(G1<V>* base, unsigned byte) {
+    return *(G1<V>*)((G1<char>*)base + byte);
+}
+template <class V> __device__ __forceinline__ const G1<V>& at(const G1<V>* base, unsigned byte) {
+    return *(const G1<V>*)((const G1<char>*)base + byte);
+}
+// A value the compiler cannot see through: addresses formed from it are recomputed at each use
+// (formed ahead of the iterations they would not fit the registers).
+__device__ __forceinline__ int opaque(int q) {
+    asm volatile("" : "+v"(q));
+    return q;
+}
+typedef float f3n __attribute__((ext_vector_type(3)));
+
+constexpr int BLK = 256;     // rows of one partial sum
+
+struct Group {
+    G1<uint64_t>* slots;
+    float* lds;   // 2 * (T / 64 + 4) floats
+    int* gaveUp;  // LDS flag: a wait of this workgroup ran out
+    int G, wg;
+    unsigned epoch;
+};
+
+// Sums v over the group; every thread of every workgroup gets the same sums.  The order of the sum is
+// that of the separate launches (cs_pcg.hip) and depends on the rows alone, not on T or on how many
+// systems share the launch: a partial per 256 rows (64 by a shuffle tree, four of those pairwise),
+// partials t, t + 256, .. to lane t of 256, and those 256 as the rows of a partial.  On return all
+// stores that any thread of the group made before the call are visible to every thread.  False if the
+// wait ran out (the same in every thread of the workgroup).  PUBLISH false: only the sums are
+// exchanged; stores made before become visible at the next meeting with PUBLISH.
+template <int T, int NS, bool PUBLISH = true>
+__device__ __forceinline__ bool meet(Group& g, float (&v)[NS]) {
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    constexpr int NW = T / 64, NB = T / BLK;  // waves, partials per workgroup
+#pragma unroll
+    for (int s = 0; s < NS; s++)
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) v[s] += __shfl_xor(v[s], o, 64);
+    if (lane == 0)
+#pragma unroll
+        for (int s = 0; s < NS; s++) g.lds[NW * s + wave] = v[s];
+    if (PUBLISH) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's published vectors are out
+    __syncthreads();
+    auto partial = [&](int s, int b) {
+        const float* w = g.lds + NW * s + 4 * b;
+        return (w[0] + w[1]) + (w[2] + w[3]);
+    };
+    if (g.G == 1) {
+#pragma unroll
+        for (int s = 0; s < NS; s++) {
+            v[s] = partial(s, 0);
+#pragma unroll
+            for (int b = 1; b < NB; b++) v[s] += partial(s, b);
+        }
+        __syncthreads();
+        return true;
+    }
+    const unsigned ep = ++g.epoch;
+    const int n = g.G * NB;  // slots per value
+    G1<uint64_t>* gen = g.slots + (ep & 1) * 2 * n;
+    if (tid < NS * NB) {
+        const int s = tid / NB, b = tid % NB;
+        put64(&at(gen, 8u * (s * n + g.wg * NB + b)), (uint64_t)ep << 32 | __float_as_uint(partial(s, b)));
+    }
+    // the 256 lanes are four waves' worth; a wave polls its lanes' slots
+    float* sums = g.lds + 2 * NW;
+    unsigned long long since = 0;
+    for (int c = wave; c < 4; c += NW) {
+        float a[NS];
+#pragma unroll
+        for (int s = 0; s < NS; s++) a[s] = 0.0f;
+        for (int t = 64 * c + lane; t < n; t += BLK) {
+            uint64_t w[NS];
+            for (int spin = 0;; spin++) {
+                bool all = true;
+#pragma unroll
+                for (int s = 0; s < NS; s++) {
+                    w[s] = get64(&at(gen, 8u * (s * n + opaque(t))));
+                    all = all && (unsigned)(w[s] >> 32) == ep;
+                }
+                if (all) break;
+                if ((spin & 1023) == 1023) {
+                    const unsigned long long now = wall_clock64();
+                    if (since == 0) since = now;
+                    if (now - since > WAIT_TICKS) {
+                        *g.gaveUp = 1;
+                        break;
+                    }
+                }
+            }
+#pragma unroll
+            for (int s = 0; s < NS; s++) a[s] += __uint_as_float((unsigned)w[s]);
+        }
+        if (64 * c < n)
+#pragma unroll
+            for (int s = 0; s < NS; s++)
+#pragma unroll
+                for (int o = 32; o > 0; o >>= 1) a[s] += __shfl_xor(a[s], o, 64);
+        if (lane == 0)
+#pragma unroll
+            for (int s = 0; s < NS; s++) sums[4 * s + c] = a[s];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int s = 0; s < NS; s++) v[s] = (sums[4 * s] + sums[4 * s + 1]) + (sums[4 * s + 2] + sums[4 * s + 3]);
+    const bool ok = *g.gaveUp == 0;
+    // vectors cached from before the meeting are dropped (one wave: the caches are the CU's and
+    // the XCD's), before any thread goes on to gather
+    if (PUBLISH && tid == 0) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+    __syncthreads();
+    return ok;
+}
+
+template <class P> __device__ __forceinline__ V3f ld3v(P p, int i) { return mk(p[3 * i], p[3 * i + 1], p[3 * i + 2]); }
+__device__ __forceinline__ V3f v3(float4 a) { return mk(a.x, a.y, a.z); }
+__device__ __forceinline__ V3f v3(f4n a) { return mk(a.x, a.y, a.z); }
+__device__ __forceinline__ V3f v3(f3n a) { return mk(a.x, a.y, a.z); }
+__device__ __forceinline__ V3f mul3(const float (&m)[9], V3f a) {
+    return mk(m[0] * a.x + m[1] * a.y + m[2] * a.z, m[3] * a.x + m[4] * a.y + m[5] * a.z,
+              m[6] * a.x + m[7] * a.y + m[8] * a.z);
+}
+// (as acc3 of cs_pcg.hip: the same operations in the same order give the same bits)
+__device__ __forceinline__ void acc3(V3f& y, const float (&a)[9], V3f v) {
+    y.x += a[0] * v.x + a[1] * v.y + a[2] * v.z;
+    y.y += a[3] * v.x + a[4] * v.y + a[5] * v.z;
+    y.z += a[6] * v.x + a[7] * v.y + a[8] * v.z;
+}
+
+// The recursive stop of a continuation (cs_pcg.hip, continuation_stop)
+__device__ __forceinline__ float continuation_stop(float tol2bb, int restarts) {
+    return restarts >= 1 ? 0.25f * tol2bb : tol2bb;
+}
+
+// 3x3 block c of a block-CSR value array: 36 B in three loads (the memory unit handles a wave's 64
+// scattered lines once per load, so nine loads of 4 B cost three times as much)
+typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
+__device__ __forceinline__ void ldblk(const G1<float>* v, unsigned k, float (&o)[9]) {
+    const G1<char>* b = (const G1<char>*)v + 36u * k;
+    const f4u p = *(const G1<f4u>*)b, q = *(const G1<f4u>*)(b + 16);
+    o[0] = p.x; o[1] = p.y; o[2] = p.z; o[3] = p.w;
+    o[4] = q.x; o[5] = q.y; o[6] = q.z; o[7] = q.w;
+    o[8] = *(const G1<float>*)(b + 32);
+}
+
+// a gathered neighbour's z and previous d
+struct Pair {
+    V3f z, d;
+};
+// One row per thread, T rows per workgroup, one 64-row slice per wave; RS slots of a row in
+// registers (interior rows of a grid have 13), any further ones read from memory every iteration;
+// the gathers of GR slots are in flight together.  LOCAL: the system has one workgroup, whose
+// vectors are exchanged through LDS.
+template <int T, int RS, int GR, bool LOCAL>
+__global__ void __launch_bounds__(T) k_ppcg(const PSys* __restrict__ tab, const int2* __restrict__ map, float tol2,
+                                            int maxit) {
+    constexpr int NW = T / 64;
+    __shared__ float red[2 * (NW + 4)];
+    __shared__ int gaveUp;
+    __shared__ float4 zl[LOCAL ? T : 1], dl[LOCAL ? T : 1];
+    const int2 m2 = map[blockIdx.x];
+    const int id = __builtin_amdgcn_readfirstlane(m2.x), wg = __builtin_amdgcn_readfirstlane(m2.y);
+    if (id < 0) return;
+    const PSysG S = gview(tab[id]);
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int nn = S.nn;
+    Group g;
+    g.slots = S.slots;
+    g.lds = red;
+    g.gaveUp = &gaveUp;
+    g.G = S.G;
+    g.wg = wg;
+    g.epoch = 0;
+    if (tid == 0) gaveUp = 0;
+
+    const V3f zero = mk(0.0f, 0.0f, 0.0f);
+    const int i = wg * T + tid, ic = min(i, nn - 1);
+    const bool live = i < nn;
+    // a slice past the last reads the last one's blocks, masked to zero (no branches around loads)
+    const int sl = min(wg * NW + wave, S.nslices - 1);
+    const int W = S.sliceW[sl];
+    const G1<int>* cb = S.cols + (size_t)S.sliceOff[sl] * SLICE;
+    const G1<float>* vb = S.vals + (size_t)S.sliceOff[sl] * 9 * SLICE;
+    float a[RS][9];
+    int rel[(RS + 1) / 2];  // two 16-bit column offsets each
+#pragma unroll
+    for (int k = 0; k < RS; k++)
+#pragma unroll
+        for (int c = 0; c < 9; c++) a[k][c] = at(vb, 4u * ((min(k, W - 1) * 9 + c) * SLICE + lane));
+#pragma unroll
+    for (int k = 0; k < RS; k++)
+#pragma unroll
+        for (int c = 0; c < 9; c++) {
+            asm volatile("" : "+v"(a[k][c]));
+            a[k][c] = k < W && live ? a[k][c] : 0.0f;
+            asm volatile("" : "+v"(a[k][c]));  // masked here and now, not where it is first used
+        }
+#pragma unroll
+    for (int k = 0; k < (RS + 1) / 2; k++) {
+        int lo = at(cb, 4u * (min(2 * k, W - 1) * SLICE + lane)) - i;
+        int hi = at(cb, 4u * (min(2 * k + 1, W - 1) * SLICE + lane)) - i;
+        asm volatile("" : "+v"(lo), "+v"(hi));
+        lo = 2 * k < W && live ? lo : 0;
+        hi = 2 * k + 1 < W && live ? hi : 0;
+        rel[k] = (lo & 0xffff) | (hi << 16);
+    }
+
+    auto row = [&]() { return opaque(ic); };
+    auto zAt = [&](int j) { return LOCAL ? v3(zl[j]) : v3(at((const G1<f3n>*)S.z, 16u * j)); };
+    auto dAt = [&](const G1<f4n>* dp, int j) { return LOCAL ? v3(dl[j]) : v3(at((const G1<f3n>*)dp, 16u * j)); };
+    // The operand of a product is formed as it is gathered, gat(column); put(block, operand) adds.
+    auto contacts = [&](auto& gat, auto& put) {
+        if (!S.contacts || !live) return;
+        const int c1 = at(S.cRowPtr, 4u * row() + 4u);
+        for (int k = at(S.cRowPtr, 4u * row()); k < c1; k++) {
+            float o[9];
+            ldblk(S.cVal, k, o);
+            put(o, gat(at(S.cCol, 4u * k)));
+        }
+    };
+    // slots k0.. of the row from memory
+    auto streamed = [&](int k0, auto& gat, auto& put) {
+        for (int k = k0; k < W; k++) {
+            float o[9];
+            const int j = at(cb, 4u * (k * SLICE + lane));
+#pragma unroll
+            for (int c = 0; c < 9; c++) o[c] = at(vb, 4u * ((k * 9 + c) * SLICE + lane));
+            put(o, gat(live ? j : ic));
+        }
+    };
+    // the pattern's slots in order, then the contacts
+    auto sweep = [&](auto& gat, auto& put) {
+        const int q = row();
+#pragma unroll
+        for (int k = 0; k < (RS + 1) / 2; k++) asm volatile("" : "+v"(rel[k]));  // columns unpacked here, not kept
+        auto col = [&](int k) { return q + ((k & 1) ? rel[k >> 1] >> 16 : (int)(short)(rel[k >> 1] & 0xffff)); };
+#pragma unroll
+        for (int k0 = 0; k0 < RS; k0 += GR) {
+            decltype(gat(0)) w[GR];
+#pragma unroll
+            for (int u = 0; u < GR; u++)
+                if (k0 + u < RS) w[u] = gat(col(k0 + u));
+#pragma unroll
+            for (int u = 0; u < GR; u++)
+                if (k0 + u < RS) put(a[k0 + u], w[u]);
+        }
+        streamed(RS, gat, put);
+        contacts(gat, put);
+    };
+    auto putZ = [&](V3f v) {
+        if (LOCAL) zl[tid] = st4(v);
+        else if (live) put3(&at(S.z, 16u * row()), v);
+    };
+    auto rhs = [&](int k) { return ld3v(&at(S.b, 12u * k), 0) + ld3v(&at(S.bc, 12u * k), 0); };
+
+    // x = 0, r = b, z = Minv r
+    float m[9];
+    ldblk(S.Minv, row(), m);
+    V3f x = zero, d = zero, q = zero, r = live ? rhs(row()) : zero, z = mul3(m, r);
+    putZ(z);
+    float v2[2] = {dot(r, z), dot(r, r)};
+    if (!meet<T, 2>(g, v2)) return;
+    float rz = v2[0], rzOld = 1.0f;
+    const float bb = v2[1], tol2bb = tol2 * bb;
+    float rr = bb, stop2bb = tol2bb;
+    bool run = !(bb <= tol2bb || maxit <= 0);
+    int it = 0;
+    for (int restarts = 0;; restarts++) {
+        for (const int first = it; run; it++) {
+            // stop on the tolerance, the budget, or a non-finite r.r (NaN fails every comparison)
+            if (it > first && (rr <= stop2bb || it >= maxit || !(rr <= FLT_MAX))) break;
+            q = zero;
+            if (it == first) {
+                auto gat = [&](int j) { return zAt(j); };
+                auto put = [&](const float (&o)[9], V3f w) { acc3(q, o, w); };
+                sweep(gat, put);
+                d = z;
+            } else {
+                const float beta = rz / rzOld;
+                const G1<f4n>* dprev = S.d + (1 - (it & 1)) * nn;
+                auto gat = [&](int j) { return Pair{zAt(j), dAt(dprev, j)}; };
+                V3f t = zero;  // q = A z + beta (A d_prev)
+                auto put = [&](const float (&o)[9], Pair w) {
+                    acc3(q, o, w.z);
+                    acc3(t, o, w.d);
+                };
+                sweep(gat, put);
+                d = mk(z.x + beta * d.x, z.y + beta * d.y, z.z + beta * d.z);
+                q = mk(q.x + beta * t.x, q.y + beta * t.y, q.z + beta * t.z);
+            }
+            if (LOCAL) {
+                __syncthreads();  // every gather of the previous d is done
+                dl[tid] = st4(d);
+            } else if (live) {
+                put3(&at(S.d + (it & 1) * nn, 16u * row()), d);
+            }
+            float v1[1] = {live ? dot(d, q) : 0.0f};
+            ldblk(S.Minv, row(), m);  // ahead of the meeting
+            if (!meet<T, 1, false>(g, v1)) return;
+            const float alpha = rz / v1[0];
+            if (live) {
+                x = x + alpha * d;
+                r = r - alpha * q;
+            }
+            z = mul3(m, r);
+            putZ(z);
+            v2[0] = dot(r, z);
+            v2[1] = dot(r, r);
+            if (!meet<T, 2>(g, v2)) return;
+            rzOld = rz;
+            rz = v2[0];
+            rr = v2[1];
+        }
+        // the true residual b - A x with every row sum in FP64, the matrix from memory (once per stop)
+        putZ(x);
+        v2[0] = v2[1] = 0.0f;
+        if (!meet<T, 2>(g, v2)) return;
+        if (live) {
+            double y0 = 0.0, y1 = 0.0, y2 = 0.0;
+            auto put = [&](const float (&o)[9], V3f xj) {
+                y0 += (double)o[0] * xj.x + (double)o[1] * xj.y + (double)o[2] * xj.z;
+                y1 += (double)o[3] * xj.x + (double)o[4] * xj.y + (double)o[5] * xj.z;
+                y2 += (double)o[6] * xj.x + (double)o[7] * xj.y + (double)o[8] * xj.z;
+            };
+            streamed(0, zAt, put);
+            contacts(zAt, put);
+            const V3f b = ld3v(&at(S.b, 12u * row()), 0), bc = ld3v(&at(S.bc, 12u * row()), 0);
+            r = mk((float)((double)b.x + (double)bc.x - y0), (float)((double)b.y + (double)bc.y - y1),
+                   (float)((double)b.z + (double)bc.z - y2));
+        }
+        ldblk(S.Minv, row(), m);
+        z = mul3(m, r);
+        v2[0] = dot(r, z);
+        v2[1] = dot(r, r);
+        if (!meet<T, 2>(g, v2)) return;
+        rz = v2[0];
+        rr = v2[1];
+        if (rr <= tol2bb || it >= maxit || !(rr <= FLT_MAX) || restarts == RESTARTS) break;
+        // continue from it, the direction restarted from z
+        stop2bb = continuation_stop(tol2bb, restarts);
+        run = true;
+        putZ(z);
+        float none[1] = {0.0f};
+        if (!meet<T, 1>(g, none)) return;
+    }
+    if (live) {
+        G1<float>* o = &at(S.x, 12u * row());
+        o[0] = x.x;
+        o[1] = x.y;
+        o[2] = x.z;
+    }
+    if (wg == 0 && tid == 0) {
+        S.out->rr = rr;
+        S.out->bb = bb;
+        S.out->tol2bb = tol2bb;
+        S.out->iters = it;
+        S.out->done = 1;
+    }
+}
+
+// A system's launch table entry: its group has G workgroups, its slots start at `slots`.
+PSys describe(const ClothSys& S, int G, uint64_t* slots, PcgScalars* out) {
+    PSys p{};
+    p.nn = S.nn;
+    p.nslices = S.nslices;
+    p.G = G;
+    p.contacts = S.nContact;
+    p.sliceOff = S.sliceOff.ptr<int>();
+    p.sliceW = S.sliceW.ptr<int>();
+    p.cols = S.cols.ptr<int>();
+    p.cRowPtr = S.cRowPtr.ptr<int>();
+    p.cCol = S.nContact > 0 ? S.cCol.ptr<int>() : p.cRowPtr;
+    p.vals = S.vals.ptr<float>();
+    p.cVal = S.nContact > 0 ? S.cVal.ptr<float>() : p.vals;
+    p.Minv = S.Minv.ptr<float>();
+    p.b = S.b.ptr<float>();
+    p.bc = S.bc.ptr<float>();
+    p.x = S.x.ptr<float>();
+    p.z = S.z.ptr<float4>();
+    p.d = S.d.ptr<float4>();
+    p.slots = slots;
+    p.out = out;
+    return p;
+}
+
+// Workgroups of T threads of kernel f the device holds at once, a multiple of 8 (0: no cooperative
+// launch): by the 512 vector registers a lane of a SIMD has for all its waves and by the LDS of a
+// CU (hipOccupancyMaxActiveBlocksPerMultiprocessor counts 256 registers).
+int resident(cs_ctx* C, const void* f, int T) {
+    int coop = 0, cus = 0, lds = 0;
+    hipFuncAttributes fa;
+    CS_HIP(hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, C->device));
+    CS_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, C->device));
+    CS_HIP(hipDeviceGetAttribute(&lds, hipDeviceAttributeMaxSharedMemoryPerMultiprocessor, C->device));
+    CS_HIP(hipFuncGetAttributes(&fa, f));
+    if (!coop || fa.numRegs <= 0) return 0;
+    const int waves = std::min(8, 512 / ((fa.numRegs + 7) & ~7));  // per SIMD
+    int per = waves * 4 / (T / 64);
+    if (fa.sharedSizeBytes > 0) per = std::min(per, (int)(lds / fa.sharedSizeBytes));
+    return (per * cus) & ~7;
+}
+
+const void* kernel_of(int T, bool local) {
+    if (local) return (const void*)k_ppcg<512, 14, 4, true>;
+    return T == 512 ? (const void*)k_ppcg<512, 14, 4, false> : (const void*)k_ppcg<256, 14, 7, false>;
+}
+
+}  // namespace
+
+// The systems of `cloths` (assembled, Minv current) by block-Jacobi PCG.  Results per entry of
+// `cloths`, as pcg_solve.  False, and nothing solved, when the systems do not fit the kernel (one of
+// more rows than the device holds at once, more than two launches' worth, a column more than
+// 32,767 away from its row) or a group gave up: the caller solves with separate launches.
+bool ppcg_solve(cs_ctx* C, const std::vector<int>& cloths, int* iters, float* relres, int* converged) {
+    if (C->ppOff) return false;
+    const int n = (int)cloths.size();
+    bool local = true;
+    int most = 0;
+    for (int c : cloths) {
+        const ClothSys& S = C->sys[c];
+        if (S.bandwidth > 32767) return false;
+        local = local && S.nn <= 512;
+        most = std::max(most, S.nn);
+    }
+    // Rows per workgroup: one workgroup and LDS for systems of 512 rows; otherwise a lone system is
+    // spread over more CUs by 256 (1,089 rows: 4.6 us an iteration with 256, 6.1 with 512), until the
+    // meeting of many workgroups costs more (65,536 rows: 12.6 us with 256, 9.1 with 512).  A batch
+    // fills the CUs anyway (32 cloths, 170,000 rows: 24.6 ms with 256, 15.9 with 512).
+    const int T = local || n > 1 || most > 96 * 256 ? 512 : 256;
+    const void* f = kernel_of(T, local);
+    const int cap = resident(C, f, T);
+    std::vector<int> G(n), order(n);
+    for (int k = 0; k < n; k++) {
+        G[k] = cdiv(C->sys[cloths[k]].nn, T);
+        order[k] = k;
+        if (((G[k] + 7) & ~7) > cap) return false;
+    }
+    // Launches of as many groups as fit, largest systems first (they iterate longest).  Workgroups are
+    // dealt to the 8 XCDs round-robin; a group of a batch goes to the least loaded XCD, whose L2 its
+    // vectors then share; a lone system of up to 8 workgroups too (1,089 rows: 4.6 against 5.0 us), a
+    // larger one is split into eighths (4,225 rows: 5.2 against 6.3 us on one XCD).  Beyond two
+    // launches the separate kernels win: they stream all matrices at once, while here each launch
+    // waits out its slowest system (340,000 rows in 48 cloths: 37.6 against 40 ms; 170,000 in 32:
+    // 15.9 against 22.5).
+    std::sort(order.begin(), order.end(), [&](int a, int b) { return G[a] != G[b] ? G[a] > G[b] : a < b; });
+    struct Round { int off, n; };
+    std::vector<Round> rounds;
+    std::vector<int2> map;
+    for (size_t at = 0; at < order.size();) {
+        std::vector<int2> xcd[8];
+        size_t deep = 0;
+        if (n == 1) {
+            const int per = G[0] <= 8 ? 8 : (G[0] + 7) / 8;
+            for (int w = 0; w < G[0]; w++) xcd[w / per].push_back(make_int2(0, w));
+            for (auto& v : xcd) deep = std::max(deep, v.size());
+            at = 1;
+        }
+        for (; at < order.size(); at++) {
+            const int k = order[at];
+            int x = 0;
+            for (int y = 1; y < 8; y++)
+                if (xcd[y].size() < xcd[x].size()) x = y;
+            // a group deeper than an XCD's share runs over all of them
+            if (xcd[x].size() + G[k] <= (size_t)cap / 8) {
+                for (int w = 0; w < G[k]; w++) xcd[x].push_back(make_int2(k, w));
+            } else if (deep == 0 && G[k] > cap / 8) {
+                for (int w = 0; w < G[k]; w++) xcd[w % 8].push_back(make_int2(k, w));
+            } else {
+                break;
+            }
+            for (auto& v : xcd) deep = std::max(deep, v.size());
+        }
+        rounds.push_back({(int)map.size(), (int)(8 * deep)});
+        for (size_t d = 0; d < deep; d++)
+            for (int y = 0; y < 8; y++) map.push_back(d < xcd[y].size() ? xcd[y][d] : make_int2(-1, 0));
+    }
+    if (rounds.size() > 2) return false;
+    hipStream_t s = C->stream;
+    std::vector<size_t> so(n);
+    size_t words = 0;
+    for (int k = 0; k < n; k++) {
+        so[k] = words;
+        words += 4 * (size_t)G[k] * (T / BLK);
+    }
+    uint64_t* slots = C->ppSlots.as<uint64_t>(words);
+    PcgScalars* out = C->bScal.as<PcgScalars>(n);
+    std::vector<PSys> tab(n);
+    for (int k = 0; k < n; k++) tab[k] = describe(C->sys[cloths[k]], G[k], slots + so[k], out + k);
+    PSys* dtab = C->ppTab.as<PSys>(n);
+    int2* dmap = C->ppMap.as<int2>(map.size());
+    PcgScalars* h = static_cast<PcgScalars*>(pinned_batch(C, sizeof(PcgScalars) * n));
+    CS_HIP(hipMemcpyAsync(dtab, tab.data(), sizeof(PSys) * n, hipMemcpyHostToDevice, s));
+    CS_HIP(hipMemcpyAsync(dmap, map.data(), sizeof(int2) * map.size(), hipMemcpyHostToDevice, s));
+    fill_u64(slots, 0, (long)words, s);
+    fill_u32(reinterpret_cast<uint32_t*>(out), 0u, (long)n * (sizeof(PcgScalars) / 4), s);
+    float tol2 = C->P.pcg_rel_tol * C->P.pcg_rel_tol;
+    int maxit = C->P.pcg_max_iters;
+    for (const Round& r : rounds) {
+        const PSys* ct = dtab;
+        const int2* cm = dmap + r.off;
+        void* args[] = {(void*)&ct, (void*)&cm, (void*)&tol2, (void*)&maxit};
+        const hipError_t e = hipLaunchCooperativeKernel(f, dim3(r.n), dim3(T), args, 0, s);
+        if (e != hipSuccess) {
+            // too large, or another process holds the device's cooperative queue
+            (void)hipGetLastError();
+            CS_HIP(hipStreamSynchronize(s));
+            C->ppOff = true;
+            return false;
+        }
+    }
+    CS_HIP(hipMemcpyAsync(h, out, sizeof(PcgScalars) * n, hipMemcpyDeviceToHost, s));
+    CS_HIP(hipStreamSynchronize(s));
+    for (int k = 0; k < n; k++)
+        if (!h[k].done) {
+            C->ppOff = true;
+            return false;
+        }
+    for (int k = 0; k < n; k++) {
+        iters[k] = h[k].iters;
+        relres[k] = h[k].bb > 0.0f ? sqrtf(h[k].rr / h[k].bb) : 0.0f;
+        converged[k] = h[k].rr <= h[k].tol2bb;
+        C->sys[cloths[k]].solved = converged[k] != 0;
+    }
+    return true;
+}
+
+}  // namespace cs

@@ -40,9 +40,11 @@ int pcg_solve(cs_ctx* C, int c, float* relres, int* converged);
 // PCG of every cloth at once (independent instances); per-cloth results.  amg: each cloth whose
 // hierarchy is usable is preconditioned by its multigrid cycle, the others by block Jacobi.
 void pcg_solve_batched(cs_ctx* C, int* iters, float* relres, int* converged, bool amg = false);
-// Block-Jacobi PCG of the listed cloths' systems, each whole solve inside one launch (cs_ppcg.hip);
-// false when they do not fit it.
-bool ppcg_solve(cs_ctx* C, const std::vector<int>& cloths, int* iters, float* relres, int* converged);
+// Whole solves inside one launch (cs_ppcg.hip), the launched iterations' results bit for bit: cloth c's
+// system (its preconditioner prepared), or every cloth's (the multigrid is prepared inside).  False
+// when they do not fit: the caller solves with separate launches.
+bool ppcg_solve(cs_ctx* C, int c, bool amg, bool learned, int* iters, float* relres, int* converged);
+bool ppcg_solve_batch(cs_ctx* C, bool amg, int* iters, float* relres, int* converged);
 // aggregation multigrid preconditioner (cs_amg.hip)
 constexpr float AMG_OMEGA = 0.6f;  // damping of the block-Jacobi smoother
 // batched multigrid of the independent cloths: bamg_build returns, per cloth, 1 if its

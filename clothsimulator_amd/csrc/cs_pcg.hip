@@ -134,6 +134,24 @@ __device__ __forceinline__ void acc3(float& y0, float& y1, float& y2, const floa
     y2 += a[6] * v.x + a[7] * v.y + a[8] * v.z;
 }
 
+// 3x3 block k of a block-CSR value array: 36 B in three loads.  The memory unit handles a wave's 64
+// scattered lines once per load, so nine loads of 4 B cost three times as much.
+typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
+__device__ __forceinline__ void ldblk(const float* __restrict__ v, int k, float (&o)[9]) {
+    const float* b = v + 9 * (size_t)k;
+    const f4u p = *(const f4u*)b, q = *(const f4u*)(b + 4);
+    o[0] = p.x; o[1] = p.y; o[2] = p.z; o[3] = p.w;
+    o[4] = q.x; o[5] = q.y; o[6] = q.z; o[7] = q.w;
+    o[8] = b[8];
+}
+__device__ __forceinline__ void ldblk(const G1<float>* v, int k, float (&o)[9]) {
+    const G1<float>* b = v + 9 * (size_t)k;
+    const f4u p = *(const G1<f4u>*)b, q = *(const G1<f4u>*)(b + 4);
+    o[0] = p.x; o[1] = p.y; o[2] = p.z; o[3] = p.w;
+    o[4] = q.x; o[5] = q.y; o[6] = q.z; o[7] = q.w;
+    o[8] = b[8];
+}
+
 // How z = M^-1 r is formed after the update of r:
 //   PC_JACOBI    z = Minv r and the r.z partials, in the same kernel;
 //   PC_SMOOTH    the multigrid cycle that follows computes z and r.z; this kernel
@@ -257,13 +275,24 @@ __global__ void __launch_bounds__(PB) k_pcg_spmv(int it, int nn, const int* __re
         }
         if (live) {
             const int ce = cRowPtr[i + 1];
-            for (int kc = cRowPtr[i]; kc < ce; kc++) {
-                const int jj = cCol[kc];
-                float a[9];
-#pragma unroll
-                for (int c = 0; c < 9; c++) a[c] = cVal[(size_t)kc * 9 + c];
-                acc3(s0, s1, s2, a, v3(g0[jj]));
-                if (!FIRST) acc3(t0, t1, t2, a, v3(dprev[jj]));
+            for (int kc = cRowPtr[i]; kc < ce; kc += 2) {  // two blocks' loads in flight
+                const int k1 = min(kc + 1, ce - 1);
+                const int j0 = cCol[kc], j1 = cCol[k1];
+                float a0[9], a1[9];
+                ldblk(cVal, kc, a0);
+                ldblk(cVal, k1, a1);
+                const float4 z0 = g0[j0], z1 = g0[j1];
+                float4 e0, e1;
+                if (!FIRST) {
+                    e0 = dprev[j0];
+                    e1 = dprev[j1];
+                }
+                acc3(s0, s1, s2, a0, v3(z0));
+                if (!FIRST) acc3(t0, t1, t2, a0, v3(e0));
+                if (kc + 1 < ce) {
+                    acc3(s0, s1, s2, a1, v3(z1));
+                    if (!FIRST) acc3(t0, t1, t2, a1, v3(e1));
+                }
             }
         }
         if (!FIRST && first_row) {
@@ -698,8 +727,7 @@ __device__ __forceinline__ void bpcg_spmv_block(const BCloth* __restrict__ cl, i
         for (int kc = c.cRowPtr[i], ce = c.cRowPtr[i + 1]; kc < ce; kc++) {
             const int jj = c.cCol[kc];
             float a[9];
-#pragma unroll
-            for (int q = 0; q < 9; q++) a[q] = c.cVal[(size_t)kc * 9 + q];
+            ldblk(c.cVal, kc, a);
             acc3(s0, s1, s2, a, v3(c.z[jj]));
             if (!FIRST) acc3(t0, t1, t2, a, v3(dprev[jj]));
         }
@@ -878,8 +906,7 @@ __global__ void __launch_bounds__(BP) k_bpcg_true(const BCloth* __restrict__ cl,
         }
         for (int kc = c.cRowPtr[i], ce = c.cRowPtr[i + 1]; kc < ce; kc++) {
             float a[9];
-#pragma unroll
-            for (int q = 0; q < 9; q++) a[q] = c.cVal[(size_t)kc * 9 + q];
+            ldblk(c.cVal, kc, a);
             sub(a, c.cCol[kc]);
         }
         const V3f ri = mk((float)y[0], (float)y[1], (float)y[2]);
@@ -958,8 +985,7 @@ __global__ void __launch_bounds__(BP) k_bpcg_post0(const BCloth* __restrict__ cl
         }
         for (int kc = c.cRowPtr[i], ce = c.cRowPtr[i + 1]; kc < ce; kc++) {
             float a[9];
-#pragma unroll
-            for (int q = 0; q < 9; q++) a[q] = c.cVal[(size_t)kc * 9 + q];
+            ldblk(c.cVal, kc, a);
             acc3(y0, y1, y2, a, ld3v(c.e1, c.agg0[c.cCol[kc]]));
         }
         const V3f xi = ld3v(c.xs, i) + ld3v(c.e1, c.agg0[i]);
@@ -1001,20 +1027,6 @@ __global__ void __launch_bounds__(BP) k_bpcg_recheck(const BCloth* __restrict__ 
 
 int pcg_solve(cs_ctx* C, int c, float* relres, int* converged) {
     ClothSys& S = C->sys[c];
-    // Block Jacobi (and a cloth too small for the multigrid it asks for) is solved inside one launch
-    // where its matrix fits the chip's registers; timed runs keep the launches they time.
-    int small[16];
-    const bool jacobi = C->P.precond == CS_PRECOND_BLOCK_JACOBI ||
-                        (C->P.precond != CS_PRECOND_LEARNED && amg_levels(C, c, small, 16) <= 1);
-    if (jacobi && !(C->P.flags & CS_FLAG_TIME_KERNELS)) {
-        int it = 0, conv = 0;
-        float rel = 0.0f;
-        if (ppcg_solve(C, {c}, &it, &rel, &conv)) {
-            if (relres) *relres = rel;
-            if (converged) *converged = conv;
-            return it;
-        }
-    }
     hipStream_t s = C->stream;
     const int nn = S.nn;
     const int nb = std::min(PMAX, (cdiv(nn, PB) + 7) & ~7);
@@ -1033,10 +1045,20 @@ int pcg_solve(cs_ctx* C, int c, float* relres, int* converged) {
     const bool amg = C->P.precond == CS_PRECOND_AMG && amg_levels(C, c, levels, 16) > 1;
     const bool learned = C->P.precond == CS_PRECOND_LEARNED;
     float* xs = nullptr;  // level-0 pre-smoothing iterate of the multigrid cycle
+    if (amg || amgl) amg_prepare(C, c, amgl);  // amgl: its single-workgroup part overlaps the network's inference
+    if (learned || amgl) lpc_prepare(C, c);
+    if (amgl) lpc_smoother_prepare(C, c);
+    // the whole solve inside one launch where the matrix fits the chip's registers
+    {
+        int it = 0, conv = 0;
+        float rel = 0.0f;
+        if (ppcg_solve(C, c, amg || amgl, learned || amgl, &it, &rel, &conv)) {
+            if (relres) *relres = rel;
+            if (converged) *converged = conv;
+            return it;
+        }
+    }
     if (amgl) {
-        amg_prepare(C, c, true);  // its single-workgroup part overlaps the network's inference
-        lpc_prepare(C, c);
-        lpc_smoother_prepare(C, c);
         xs = amg_level0_x(C, c);
         hipLaunchKernelGGL(k_pcg_init<PC_EXTERNAL>, dim3(nb), dim3(PB), 0, s, nn, S.b.ptr<float>(),
                            S.bc.ptr<float>(), S.Minv.ptr<float>(), S.x.ptr<float>(), S.r.ptr<float>(), z, xs, part);
@@ -1045,14 +1067,12 @@ int pcg_solve(cs_ctx* C, int c, float* relres, int* converged) {
         amg_join(C);
         amg_apply(C, c, S.r.ptr<float>(), z, part + P_RZ0 * PMAX, nb, true, true);
     } else if (amg) {
-        amg_prepare(C, c);
         xs = amg_level0_x(C, c);
         hipLaunchKernelGGL(k_pcg_init<PC_SMOOTH>, dim3(nb), dim3(PB), 0, s, nn, S.b.ptr<float>(), S.bc.ptr<float>(),
                            S.Minv.ptr<float>(), S.x.ptr<float>(), S.r.ptr<float>(), z, xs, part);
         CS_LAUNCH_CHECK();
         amg_apply(C, c, S.r.ptr<float>(), z, part + P_RZ0 * PMAX, nb, true);
     } else if (learned) {
-        lpc_prepare(C, c);
         hipLaunchKernelGGL(k_pcg_init<PC_EXTERNAL>, dim3(nb), dim3(PB), 0, s, nn, S.b.ptr<float>(),
                            S.bc.ptr<float>(), S.Minv.ptr<float>(), S.x.ptr<float>(), S.r.ptr<float>(), z, xs, part);
         CS_LAUNCH_CHECK();
@@ -1461,12 +1481,9 @@ void pcg_solve_batched(cs_ctx* C, int* iters, float* relres, int* converged, boo
     else if (tuning) cand = T.trials % kTuneN;
     const auto t0 = std::chrono::steady_clock::now();
     const int chunk = amg ? kTuneChunk[cand] / 4 : kTuneChunk[cand];
-    // block Jacobi: every cloth's whole solve inside one or two launches where the matrices fit the
-    // chip (no candidate applies there: a cloth's result is that of its own single solve, bit for
-    // bit); timed runs keep the launches they time
-    std::vector<int> every(C->nCloths);
-    for (int c = 0; c < C->nCloths; c++) every[c] = c;
-    const bool onchip = !amg && !(C->P.flags & CS_FLAG_TIME_KERNELS) && ppcg_solve(C, every, iters, relres, converged);
+    // every cloth's whole solve inside one or two launches where the matrices fit the chip (no
+    // candidate applies there: the results are those of 256 rows, bit for bit)
+    const bool onchip = ppcg_solve_batch(C, amg, iters, relres, converged);
     if (onchip) {
     } else if (kTuneRows[cand] == 128) solve_batched<128>(C, chunk, iters, relres, converged, amg);
     else solve_batched<256>(C, chunk, iters, relres, converged, amg);

@@ -1,4 +1,4 @@
-// cs_ppcg.hip — block-Jacobi PCG of whole systems in one launch, the matrix held in registers.
+// cs_ppcg.hip — PCG of whole systems in one launch, the matrix held in registers.
 //
 // A separately launched iteration (cs_pcg.hip) of a system of 16,641 rows or fewer takes 13-14 us,
 // nearly all of it latency: two kernel boundaries, and in each kernel a chain of dependent loads.
@@ -23,13 +23,21 @@
 // refused, and if a wait (each is bounded in time) runs out, the context solves with separate
 // launches from then on.
 //
-// Measured (solve time per iteration, separate launches -> here): 289 rows 14.1 -> 2.8 us,
+// The preconditioner is part of the kernel: block Jacobi in the update; the learned factor's two
+// sweeps; or the multigrid cycle with the rows of each coarse level spread over the group's waves, a
+// meeting per phase (restriction, pre-smoothing with residual, post-smoothing) instead of a launch.
+//
+// Measured (block Jacobi, solve time per iteration, separate launches -> here): 289 rows 14.1 -> 2.8 us,
 // 1,089 rows 13.5 -> 4.6, 16,641 rows with contacts 13.6 -> 7.9, 32,761 rows 13.9 -> 7.1,
 // 65,536 rows 18.0 -> 9.1, 129,600 rows 21.6 -> 15.3.
+// Solves with their set-up: learned factor 1,089 rows 3.9 -> 2.6 ms, 16,384 rows 9.0 -> 7.8, 32,400 rows
+// 9.5 -> 6.6; multigrid 289 rows 1.2 -> 0.8 ms, 4,225 rows 4.3 -> 3.6, 16,641 rows in contact 7.2 -> 5.8,
+// 32,400 rows 5.1 -> 3.6, 65,536 rows 7.4 -> 5.9.
 #include <algorithm>
 #include <cfloat>
 #include <cmath>
 #include <cstring>
+#include <type_traits>
 
 #include "cs_kernels.hpp"
 #include "cs_math.hpp"
@@ -38,8 +46,19 @@ namespace cs {
 
 namespace {
 
+enum { PRE_JACOBI = 0, PRE_LEARNED = 1, PRE_AMG = 2 };
 constexpr int RESTARTS = 4;                      // continuations from the true residual, as pcg_solve
 constexpr unsigned long long WAIT_TICKS = 200000000ull;  // 2 s of the 100 MHz wall clock
+
+// One level of a cloth's multigrid hierarchy (cs_amg.hip); agg, mptr, midx lead to the next level.
+struct PLev {
+    int n, pad;
+    const int *rp, *ci, *agg, *mptr, *midx;
+    const float *val, *Dinv;
+    float *b, *x, *t;  // right-hand side, pre-smoothed iterate, residual and then result
+};
+constexpr int MAXL = 12;
+constexpr int BOTTOM = 512;  // nodes of the level solved by a dense operator, at most
 
 struct PSys {
     int nn, nslices, G, contacts;
@@ -49,6 +68,17 @@ struct PSys {
     float4 *z, *d;      // z: nn, d: two generations of nn
     uint64_t* slots;    // 2 generations x 2 values x (G * T / BLK) words (epoch << 32 | value), zero at launch
     PcgScalars* out;
+    // learned factor: bf16 blocks in the value layout, diagonal slot and length of each row, y = G r
+    const int *diagSlot, *rowLen;
+    const uint16_t* Gf;
+    float4* y;
+    // multigrid: levels 0 .. bottom, the bottom's dense operator (3 n rows) and result, level 0's A P
+    int bottom, pad2;
+    const float* op;
+    float* eBottom;
+    const int *apSliceOff, *apSliceW, *apCols;
+    const float* apVals;
+    PLev L[MAXL];
 };
 
 // The pointers in the global address space (cs_math.hpp, G1)
@@ -60,6 +90,9 @@ struct PSysG {
     G1<f4n> *z, *d;
     G1<uint64_t>* slots;
     PcgScalars* out;
+    const G1<int> *diagSlot, *rowLen;
+    const G1<uint16_t>* Gf;
+    G1<f4n>* y;
 };
 __device__ __forceinline__ PSysG gview(const PSys& c) {
     PSysG g;
@@ -75,6 +108,26 @@ __device__ __forceinline__ PSysG gview(const PSys& c) {
     g.d = (G1<f4n>*)c.d;
     g.slots = g1(c.slots);
     g.out = c.out;
+    g.diagSlot = g1(c.diagSlot);
+    g.rowLen = g1(c.rowLen);
+    g.Gf = g1(c.Gf);
+    g.y = (G1<f4n>*)c.y;
+    return g;
+}
+
+// A level's pointers in the global address space
+struct PLevG {
+    int n;
+    const G1<int> *rp, *ci, *agg, *mptr, *midx;
+    const G1<float> *val, *Dinv;
+    G1<float> *b, *x, *t;
+};
+__device__ __forceinline__ PLevG gview(const PLev& c) {
+    PLevG g;
+    g.n = c.n;
+    g.rp = g1(c.rp); g.ci = g1(c.ci); g.agg = g1(c.agg); g.mptr = g1(c.mptr); g.midx = g1(c.midx);
+    g.val = g1(c.val); g.Dinv = g1(c.Dinv);
+    g.b = g1(c.b); g.x = g1(c.x); g.t = g1(c.t);
     return g;
 }
 
@@ -89,6 +142,13 @@ __device__ __forceinline__ void put3(G1<f4n>* p, V3f a) {
     G1<uint64_t>* q = (G1<uint64_t>*)p;
     put64(q, (uint64_t)__float_as_uint(a.y) << 32 | __float_as_uint(a.x));
     put64(q + 1, __float_as_uint(a.z));
+}
+
+// the same into an array of three floats a row
+__device__ __forceinline__ void put3f(G1<float>* p, V3f a) {
+    __hip_atomic_store(p, a.x, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(p + 1, a.y, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(p + 2, a.z, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
 // Element at a 32-bit byte offset from a uniform base: one scalar base and one offset register
@@ -124,7 +184,7 @@ struct Group {
 // stores that any thread of the group made before the call are visible to every thread.  False if the
 // wait ran out (the same in every thread of the workgroup).  PUBLISH false: only the sums are
 // exchanged; stores made before become visible at the next meeting with PUBLISH.
-template <int T, int NS, bool PUBLISH = true>
+template <int T, int NS, bool PUBLISH = true, bool LOCAL = false>
 __device__ __forceinline__ bool meet(Group& g, float (&v)[NS]) {
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     constexpr int NW = T / 64, NB = T / BLK;  // waves, partials per workgroup
@@ -148,6 +208,7 @@ __device__ __forceinline__ bool meet(Group& g, float (&v)[NS]) {
 #pragma unroll
             for (int b = 1; b < NB; b++) v[s] += partial(s, b);
         }
+        if (PUBLISH && !LOCAL && tid == 0) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
         __syncthreads();
         return true;
     }
@@ -238,6 +299,69 @@ __device__ __forceinline__ void ldblk(const G1<float>* v, unsigned k, float (&o)
     o[8] = *(const G1<float>*)(b + 32);
 }
 
+// ---- rows of the coarse levels (block CSR), the operations and order of cs_amg.hip's kernels
+
+// sum of t over the members of aggregate I (ascending)
+__device__ __forceinline__ V3f restricted(int I, const G1<int>* mptr, const G1<int>* midx, const G1<float>* t) {
+    V3f s = mk(0.0f, 0.0f, 0.0f);
+    const int k0 = at(mptr, 4u * I), k1 = at(mptr, 4u * I + 4u);
+    for (int k = k0; k < k1; k += 8) {  // eight members' loads at a time, summed in order
+        V3f m[8];
+#pragma unroll
+        for (int u = 0; u < 8; u++) m[u] = ld3v(&at(t, 12u * at(midx, 4u * min(k + u, k1 - 1))), 0);
+#pragma unroll
+        for (int u = 0; u < 8; u++)
+            if (k + u < k1) s = s + m[u];
+    }
+    return s;
+}
+
+// f(block, column) gives the operand of each block of row i; the sum over the blocks in order, the
+// loads of NB blocks in flight together
+template <int NB, class F>
+__device__ __forceinline__ V3f blockrow(int i, const G1<int>* rp, const G1<int>* ci, const G1<float>* val, F&& f) {
+    V3f y = mk(0.0f, 0.0f, 0.0f);
+    const int k0 = at(rp, 4u * i), k1 = at(rp, 4u * i + 4u);
+    for (int k = k0; k < k1; k += NB) {
+        float a[NB][9];
+        V3f w[NB];
+#pragma unroll
+        for (int u = 0; u < NB; u++) {
+            const int kk = min(k + u, k1 - 1);
+            ldblk(val, kk, a[u]);
+            w[u] = f(at(ci, 4u * kk));
+        }
+#pragma unroll
+        for (int u = 0; u < NB; u++)
+            if (k + u < k1) acc3(y, a[u], w[u]);
+    }
+    return y;
+}
+
+// x = w D^-1 b (formed on the fly for the gathered rows) and t = b - A x
+__device__ __forceinline__ void presmoothed(int i, const G1<int>* rp, const G1<int>* ci, const G1<float>* val,
+                                            const G1<float>* Dinv, const G1<float>* b, V3f& x, V3f& t) {
+    auto pre = [&](int j) {
+        float o[9];
+        ldblk(Dinv, j, o);
+        return AMG_OMEGA * mul3(o, ld3v(&at(b, 12u * j), 0));
+    };
+    const V3f y = blockrow<3>(i, rp, ci, val, pre);
+    x = pre(i);
+    t = ld3v(&at(b, 12u * i), 0) - y;
+}
+
+// x' + w D^-1 (b - A x'), x' = x + e_agg
+__device__ __forceinline__ V3f postsmoothed(int i, const G1<int>* rp, const G1<int>* ci, const G1<float>* val,
+                                            const G1<float>* Dinv, const G1<int>* agg, const G1<float>* e,
+                                            const G1<float>* b, const G1<float>* x) {
+    auto pro = [&](int j) { return ld3v(&at(x, 12u * j), 0) + ld3v(&at(e, 12u * at(agg, 4u * j)), 0); };
+    const V3f y = blockrow<3>(i, rp, ci, val, pro);
+    float o[9];
+    ldblk(Dinv, i, o);
+    return pro(i) + AMG_OMEGA * mul3(o, ld3v(&at(b, 12u * i), 0) - y);
+}
+
 // a gathered neighbour's z and previous d
 struct Pair {
     V3f z, d;
@@ -245,18 +369,21 @@ struct Pair {
 // One row per thread, T rows per workgroup, one 64-row slice per wave; RS slots of a row in
 // registers (interior rows of a grid have 13), any further ones read from memory every iteration;
 // the gathers of GR slots are in flight together.  LOCAL: the system has one workgroup, whose
-// vectors are exchanged through LDS.
-template <int T, int RS, int GR, bool LOCAL>
-__global__ void __launch_bounds__(T) k_ppcg(const PSys* __restrict__ tab, const int2* __restrict__ map, float tol2,
-                                            int maxit) {
-    constexpr int NW = T / 64;
+// vectors are exchanged through LDS.  PRE: the preconditioner, as in the separate launches.
+template <int T, int RS, int GR, bool LOCAL, int PRE>
+__global__ void __launch_bounds__(T, 2)  // 256 registers: the runtime refuses cooperative kernels of more
+    k_ppcg(const PSys* __restrict__ tab, const int2* __restrict__ map, float tol2, int maxit) {
+    constexpr int NW = T / 64, CN = 2;
     __shared__ float red[2 * (NW + 4)];
     __shared__ int gaveUp;
     __shared__ float4 zl[LOCAL ? T : 1], dl[LOCAL ? T : 1];
+    constexpr bool NET = PRE == PRE_LEARNED;
+    __shared__ float lb[PRE == PRE_AMG ? 3 * BOTTOM : 1];  // the bottom level's right-hand side
     const int2 m2 = map[blockIdx.x];
     const int id = __builtin_amdgcn_readfirstlane(m2.x), wg = __builtin_amdgcn_readfirstlane(m2.y);
     if (id < 0) return;
-    const PSysG S = gview(tab[id]);
+    const PSys& P = tab[id];
+    const PSysG S = gview(P);
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int nn = S.nn;
     Group g;
@@ -307,14 +434,23 @@ __global__ void __launch_bounds__(T) k_ppcg(const PSys* __restrict__ tab, const 
     auto contacts = [&](auto& gat, auto& put) {
         if (!S.contacts || !live) return;
         const int c1 = at(S.cRowPtr, 4u * row() + 4u);
-        for (int k = at(S.cRowPtr, 4u * row()); k < c1; k++) {
-            float o[9];
-            ldblk(S.cVal, k, o);
-            put(o, gat(at(S.cCol, 4u * k)));
+        for (int k = at(S.cRowPtr, 4u * row()); k < c1; k += CN) {  // CN blocks' loads in flight
+            float o[CN][9];
+            decltype(gat(0)) w[CN];
+#pragma unroll
+            for (int u = 0; u < CN; u++) {
+                const int kk = min(k + u, c1 - 1);
+                ldblk(S.cVal, kk, o[u]);
+                w[u] = gat(at(S.cCol, 4u * kk));
+            }
+#pragma unroll
+            for (int u = 0; u < CN; u++)
+                if (k + u < c1) put(o[u], w[u]);
         }
     };
     // slots k0.. of the row from memory
     auto streamed = [&](int k0, auto& gat, auto& put) {
+#pragma unroll 2
         for (int k = k0; k < W; k++) {
             float o[9];
             const int j = at(cb, 4u * (k * SLICE + lane));
@@ -348,22 +484,207 @@ __global__ void __launch_bounds__(T) k_ppcg(const PSys* __restrict__ tab, const 
     };
     auto rhs = [&](int k) { return ld3v(&at(S.b, 12u * k), 0) + ld3v(&at(S.bc, 12u * k), 0); };
 
-    // x = 0, r = b, z = Minv r
     float m[9];
+    V3f x = zero, d = zero, q = zero, z = zero, r = live ? rhs(row()) : zero;
+    float v1[1], v2[2], rz = 0.0f, rzOld = 1.0f, rr = 0.0f, stop2bb = -1.0f;
+    int it = 0, first = 0;
+
+    // y = G u (lower slots and the diagonal) and w = G^T u (diagonal transposed, upper slots hold the
+    // transposed lower blocks), u gathered from p: k_lpc_lower and k_lpc_upper
+    const int kd = NET ? S.diagSlot[ic] : 0, rl = NET ? S.rowLen[ic] : 0;
+    auto factor = [&](int k, float (&o)[9]) {
+        const G1<uint16_t>* gb = S.Gf + (size_t)S.sliceOff[sl] * 9 * SLICE;
+#pragma unroll
+        for (int c = 0; c < 9; c++) o[c] = __uint_as_float((unsigned)at(gb, 2u * ((k * 9 + c) * SLICE + lane)) << 16);
+    };
+    auto lower = [&](const G1<f4n>* p) {
+        V3f y = zero;
+#pragma unroll 4
+        for (int k = 0; k <= kd; k++) {
+            float o[9];
+            factor(k, o);
+            acc3(y, o, v3(at((const G1<f3n>*)p, 16u * at(cb, 4u * (k * SLICE + lane)))));
+        }
+        return y;
+    };
+    auto upper = [&](const G1<f4n>* p, V3f own) {
+        float o[9];
+        factor(kd, o);
+        V3f y = mk(o[0] * own.x + o[3] * own.y + o[6] * own.z, o[1] * own.x + o[4] * own.y + o[7] * own.z,
+                   o[2] * own.x + o[5] * own.y + o[8] * own.z);
+#pragma unroll 4
+        for (int k = kd + 1; k < rl; k++) {
+            factor(k, o);
+            acc3(y, o, v3(at((const G1<f3n>*)p, 16u * at(cb, 4u * (k * SLICE + lane)))));
+        }
+        return y;
+    };
+    auto putF = [&](G1<f4n>* p, V3f v) {
+        if (live) put3(&at(p, 16u * row()), v);
+    };
+    // G^T G u for u published in S.z by every thread
+    auto sweeps = [&](V3f& out) {
+        const V3f y = live ? lower(S.z) : zero;
+        putF(S.y, y);
+        float none[1] = {0.0f};
+        if (!meet<T, 1>(g, none)) return false;
+        out = live ? upper(S.y, y) : zero;
+        return true;
+    };
+
+    // z = M^-1 r, rz and rr of the current r; the stop test of the next iteration comes as soon as rr
+    // is known, and z is then left alone.  False: a wait ran out.
+    bool stop = false;
+    auto precondition = [&](bool test) {
+        auto stopped = [&]() {  // on the tolerance, the budget, or a non-finite r.r (NaN fails every comparison)
+            stop = test && (rr <= stop2bb || it >= maxit || !(rr <= FLT_MAX));
+            return stop;
+        };
+        if (PRE == PRE_JACOBI) {
+            z = mul3(m, r);
+            putZ(z);
+            v2[0] = dot(r, z);
+            v2[1] = dot(r, r);
+            if (!meet<T, 2, true, LOCAL>(g, v2)) return false;
+            rz = v2[0];
+            rr = v2[1];
+            stopped();
+            return true;
+        }
+        V3f xs = zero;
+        if (PRE == PRE_AMG) {
+            const V3f mr = mul3(m, r);
+            xs = mk(AMG_OMEGA * mr.x, AMG_OMEGA * mr.y, AMG_OMEGA * mr.z);
+            putF(S.z, xs);
+        } else {
+            putF(S.z, r);
+        }
+        v1[0] = dot(r, r);
+        if (!meet<T, 1>(g, v1)) return false;
+        rr = v1[0];
+        if (stopped()) return true;
+        if (PRE == PRE_LEARNED) {
+            if (!sweeps(z)) return false;
+        } else {
+            float none[1];
+            // level 0: t = r - A xs
+            V3f t = zero;
+            auto gat = [&](int j) { return zAt(j); };
+            auto put = [&](const float (&o)[9], V3f v) { acc3(t, o, v); };
+            sweep(gat, put);
+            t = r - t;
+            if (live) put3f(&at(gview(P.L[0]).t, 12u * row()), t);
+            none[0] = 0.0f;
+            if (!meet<T, 1>(g, none)) return false;
+            // down: restriction, then pre-smoothing and residual; rows in 64s over the workgroups
+            const int gr = (wave * g.G + wg) * 64 + lane, gs = g.G * T;
+            const int bottom = P.bottom;
+            for (int l = 1; l < bottom; l++) {
+                const PLevG F = gview(P.L[l - 1]), L = gview(P.L[l]);
+                for (int k = gr; k < L.n; k += gs) put3f(&at(L.b, 12u * k), restricted(k, F.mptr, F.midx, F.t));
+                none[0] = 0.0f;
+                if (!meet<T, 1>(g, none)) return false;
+                for (int k = gr; k < L.n; k += gs) {
+                    V3f xk, tk;
+                    presmoothed(k, L.rp, L.ci, L.val, L.Dinv, L.b, xk, tk);
+                    put3f(&at(L.x, 12u * k), xk);
+                    put3f(&at(L.t, 12u * k), tk);
+                }
+                none[0] = 0.0f;
+                if (!meet<T, 1>(g, none)) return false;
+            }
+            // the bottom: every workgroup restricts its whole right-hand side, a wave per row of the operator
+            {
+                const PLevG F = gview(P.L[bottom - 1]);
+                const int n = P.L[bottom].n, dim = 3 * n;
+                for (int k = tid; k < n; k += T) {
+                    const V3f b = restricted(k, F.mptr, F.midx, F.t);
+                    lb[3 * k] = b.x;
+                    lb[3 * k + 1] = b.y;
+                    lb[3 * k + 2] = b.z;
+                }
+                __syncthreads();
+                const G1<float>* op = g1(P.op);
+                G1<float>* e = g1(P.eBottom);
+                // a wave's rows of the operator, RU of them in flight together
+                auto rows = [&](auto ru) {
+                    constexpr int RU = decltype(ru)::value;
+                    for (int k = (wave * g.G + wg) * RU; k < dim; k += NW * g.G * RU) {
+                        float s[RU];
+#pragma unroll
+                        for (int u = 0; u < RU; u++) s[u] = 0.0f;
+#pragma unroll 4
+                        for (int c = lane; c < dim; c += 64) {
+                            const float v = lb[c];
+#pragma unroll
+                            for (int u = 0; u < RU; u++) s[u] += at(op, 4u * (min(k + u, dim - 1) * dim + c)) * v;
+                        }
+#pragma unroll
+                        for (int u = 0; u < RU; u++) {
+#pragma unroll
+                            for (int o = 32; o > 0; o >>= 1) s[u] += __shfl_xor(s[u], o, 64);
+                            if (lane == 0 && k + u < dim)
+                                __hip_atomic_store(&at(e, 4u * (k + u)), s[u], __ATOMIC_RELAXED,
+                                                   __HIP_MEMORY_SCOPE_AGENT);
+                        }
+                    }
+                };
+                if (dim <= NW * g.G) rows(std::integral_constant<int, 1>{});
+                else if (dim <= 2 * NW * g.G) rows(std::integral_constant<int, 2>{});
+                else if (dim <= 3 * NW * g.G) rows(std::integral_constant<int, 3>{});
+                else rows(std::integral_constant<int, 4>{});
+                none[0] = 0.0f;
+                if (!meet<T, 1>(g, none)) return false;
+            }
+            // up: prolongation and post-smoothing, a level's result into its t
+            const G1<float>* e = g1(P.eBottom);
+            for (int l = bottom - 1; l >= 1; l--) {
+                const PLevG L = gview(P.L[l]);
+                for (int k = gr; k < L.n; k += gs)
+                    put3f(&at(L.t, 12u * k), postsmoothed(k, L.rp, L.ci, L.val, L.Dinv, L.agg, e, L.b, L.x));
+                e = L.t;
+                none[0] = 0.0f;
+                if (!meet<T, 1>(g, none)) return false;
+            }
+            // level 0: the residual after the correction is t - (A P) e
+            const PLevG L = gview(P.L[0]);
+            V3f y = zero;
+            if (live) {
+                const int WA = P.apSliceW[sl];
+                const G1<int>* ac = g1(P.apCols) + (size_t)P.apSliceOff[sl] * SLICE;
+                const G1<float>* av = g1(P.apVals) + (size_t)P.apSliceOff[sl] * 9 * SLICE;
+#pragma unroll 4
+                for (int k = 0; k < WA; k++) {
+                    float o[9];
+#pragma unroll
+                    for (int c = 0; c < 9; c++) o[c] = at(av, 4u * ((k * 9 + c) * SLICE + lane));
+                    acc3(y, o, ld3v(&at(e, 12u * at(ac, 4u * (k * SLICE + lane))), 0));
+                }
+                auto gatE = [&](int j) { return ld3v(&at(e, 12u * at(L.agg, 4u * j)), 0); };
+                auto putE = [&](const float (&o)[9], V3f v) { acc3(y, o, v); };
+                contacts(gatE, putE);
+                xs = xs + ld3v(&at(e, 12u * at(L.agg, 4u * row())), 0);
+            }
+            y = t - y;
+            ldblk(S.Minv, row(), m);
+            const V3f my = mul3(m, y);
+            z = live ? mk(xs.x + AMG_OMEGA * my.x, xs.y + AMG_OMEGA * my.y, xs.z + AMG_OMEGA * my.z) : zero;
+        }
+        putF(S.z, z);
+        v1[0] = live ? dot(r, z) : 0.0f;
+        if (!meet<T, 1>(g, v1)) return false;
+        rz = v1[0];
+        return true;
+    };
+
+    // x = 0, r = b
     ldblk(S.Minv, row(), m);
-    V3f x = zero, d = zero, q = zero, r = live ? rhs(row()) : zero, z = mul3(m, r);
-    putZ(z);
-    float v2[2] = {dot(r, z), dot(r, r)};
-    if (!meet<T, 2>(g, v2)) return;
-    float rz = v2[0], rzOld = 1.0f;
-    const float bb = v2[1], tol2bb = tol2 * bb;
-    float rr = bb, stop2bb = tol2bb;
-    bool run = !(bb <= tol2bb || maxit <= 0);
-    int it = 0;
+    if (!precondition(false)) return;
+    const float bb = rr, tol2bb = tol2 * bb;
+    stop2bb = tol2bb;
+    stop = bb <= tol2bb || maxit <= 0;
     for (int restarts = 0;; restarts++) {
-        for (const int first = it; run; it++) {
-            // stop on the tolerance, the budget, or a non-finite r.r (NaN fails every comparison)
-            if (it > first && (rr <= stop2bb || it >= maxit || !(rr <= FLT_MAX))) break;
+        for (first = it; !stop;) {
             q = zero;
             if (it == first) {
                 auto gat = [&](int j) { return zAt(j); };
@@ -389,27 +710,22 @@ __global__ void __launch_bounds__(T) k_ppcg(const PSys* __restrict__ tab, const 
             } else if (live) {
                 put3(&at(S.d + (it & 1) * nn, 16u * row()), d);
             }
-            float v1[1] = {live ? dot(d, q) : 0.0f};
-            ldblk(S.Minv, row(), m);  // ahead of the meeting
-            if (!meet<T, 1, false>(g, v1)) return;
+            v1[0] = live ? dot(d, q) : 0.0f;
+            if (PRE == PRE_JACOBI || PRE == PRE_AMG) ldblk(S.Minv, row(), m);  // ahead of the meeting
+            if (!meet<T, 1, false, LOCAL>(g, v1)) return;
             const float alpha = rz / v1[0];
             if (live) {
                 x = x + alpha * d;
                 r = r - alpha * q;
             }
-            z = mul3(m, r);
-            putZ(z);
-            v2[0] = dot(r, z);
-            v2[1] = dot(r, r);
-            if (!meet<T, 2>(g, v2)) return;
+            it++;
             rzOld = rz;
-            rz = v2[0];
-            rr = v2[1];
+            if (!precondition(true)) return;
         }
         // the true residual b - A x with every row sum in FP64, the matrix from memory (once per stop)
         putZ(x);
-        v2[0] = v2[1] = 0.0f;
-        if (!meet<T, 2>(g, v2)) return;
+        v1[0] = 0.0f;
+        if (!meet<T, 1, true, LOCAL>(g, v1)) return;
         if (live) {
             double y0 = 0.0, y1 = 0.0, y2 = 0.0;
             auto put = [&](const float (&o)[9], V3f xj) {
@@ -423,20 +739,15 @@ __global__ void __launch_bounds__(T) k_ppcg(const PSys* __restrict__ tab, const 
             r = mk((float)((double)b.x + (double)bc.x - y0), (float)((double)b.y + (double)bc.y - y1),
                    (float)((double)b.z + (double)bc.z - y2));
         }
-        ldblk(S.Minv, row(), m);
-        z = mul3(m, r);
-        v2[0] = dot(r, z);
-        v2[1] = dot(r, r);
-        if (!meet<T, 2>(g, v2)) return;
-        rz = v2[0];
-        rr = v2[1];
+        v1[0] = dot(r, r);
+        if (!meet<T, 1, true, LOCAL>(g, v1)) return;
+        rr = v1[0];
         if (rr <= tol2bb || it >= maxit || !(rr <= FLT_MAX) || restarts == RESTARTS) break;
-        // continue from it, the direction restarted from z
+        // continue from it, the direction restarted from its preconditioned residual
         stop2bb = continuation_stop(tol2bb, restarts);
-        run = true;
-        putZ(z);
-        float none[1] = {0.0f};
-        if (!meet<T, 1>(g, none)) return;
+        stop = false;
+        ldblk(S.Minv, row(), m);
+        if (!precondition(false)) return;
     }
     if (live) {
         G1<float>* o = &at(S.x, 12u * row());
@@ -454,7 +765,8 @@ __global__ void __launch_bounds__(T) k_ppcg(const PSys* __restrict__ tab, const 
 }
 
 // A system's launch table entry: its group has G workgroups, its slots start at `slots`.
-PSys describe(const ClothSys& S, int G, uint64_t* slots, PcgScalars* out) {
+// dense: the multigrid's bottom is the small levels' operator, otherwise the coarsest level's inverse
+PSys describe(const ClothSys& S, int pre, bool dense, int G, uint64_t* slots, PcgScalars* out) {
     PSys p{};
     p.nn = S.nn;
     p.nslices = S.nslices;
@@ -475,6 +787,37 @@ PSys describe(const ClothSys& S, int G, uint64_t* slots, PcgScalars* out) {
     p.d = S.d.ptr<float4>();
     p.slots = slots;
     p.out = out;
+    if (pre == PRE_LEARNED) {
+        p.diagSlot = S.diagSlot.ptr<int>();
+        p.rowLen = S.rowLen.ptr<int>();
+        p.Gf = S.lpc.G.ptr<uint16_t>();
+        p.y = S.lpc.y.ptr<float4>();
+    }
+    if (pre == PRE_AMG) {
+        const AmgSys& A = S.amg;
+        p.bottom = dense ? A.smallL0 : A.nl - 1;
+        p.op = dense ? A.smallOp.ptr<float>() : A.inv.ptr<float>();
+        p.eBottom = A.L[p.bottom].t.ptr<float>();
+        p.apSliceOff = A.apSliceOff.ptr<int>();
+        p.apSliceW = A.apSliceW.ptr<int>();
+        p.apCols = A.apCols.ptr<int>();
+        p.apVals = A.apVals.ptr<float>();
+        for (int l = 0; l <= p.bottom; l++) {
+            const AmgLevel& L = A.L[l];
+            PLev& q = p.L[l];
+            q.n = L.n;
+            q.rp = L.rp.ptr<int>();
+            q.ci = L.ci.ptr<int>();
+            q.agg = L.agg.ptr<int>();
+            q.mptr = L.mptr.ptr<int>();
+            q.midx = L.midx.ptr<int>();
+            q.val = L.val.ptr<float>();
+            q.Dinv = L.Dinv.ptr<float>();
+            q.b = L.b.ptr<float>();
+            q.x = L.x.ptr<float>();
+            q.t = L.t.ptr<float>();
+        }
+    }
     return p;
 }
 
@@ -495,40 +838,77 @@ int resident(cs_ctx* C, const void* f, int T) {
     return (per * cus) & ~7;
 }
 
-const void* kernel_of(int T, bool local) {
-    if (local) return (const void*)k_ppcg<512, 14, 4, true>;
-    return T == 512 ? (const void*)k_ppcg<512, 14, 4, false> : (const void*)k_ppcg<256, 14, 7, false>;
+template <int PRE> const void* kernel_of(int T) {
+    constexpr int GR = PRE == PRE_LEARNED ? 4 : 7;  // without spilling
+    return T == 512 ? (const void*)k_ppcg<512, 14, 4, false, PRE> : (const void*)k_ppcg<256, 14, GR, false, PRE>;
+}
+const void* kernel_of(int T, bool local, int pre) {
+    if (local) return (const void*)k_ppcg<512, 14, 4, true, PRE_JACOBI>;
+    return pre == PRE_JACOBI ? kernel_of<PRE_JACOBI>(T)
+         : pre == PRE_LEARNED ? kernel_of<PRE_LEARNED>(T) : kernel_of<PRE_AMG>(T);
 }
 
-}  // namespace
+struct Round {
+    int off, n;  // its blocks in the map
+};
+struct Plan {
+    bool fits = false;
+    int T = 0;
+    const void* f = nullptr;
+    std::vector<int> G;  // workgroups per system
+    std::vector<Round> rounds;
+    std::vector<int2> map;  // block -> (system, workgroup), -1: none
+};
 
-// The systems of `cloths` (assembled, Minv current) by block-Jacobi PCG.  Results per entry of
-// `cloths`, as pcg_solve.  False, and nothing solved, when the systems do not fit the kernel (one of
-// more rows than the device holds at once, more than two launches' worth, a column more than
-// 32,767 away from its row) or a group gave up: the caller solves with separate launches.
-bool ppcg_solve(cs_ctx* C, const std::vector<int>& cloths, int* iters, float* relres, int* converged) {
-    if (C->ppOff) return false;
+// The launches for the systems of `cloths`; fits = false when one has more rows than the device holds
+// at once, a column more than 32,767 away from its row or too deep a hierarchy, or when the
+// separate launches are faster.
+Plan plan_for(cs_ctx* C, const std::vector<int>& cloths, int pre, bool dense) {
+    Plan p;
     const int n = (int)cloths.size();
-    bool local = true;
+    bool local = pre == PRE_JACOBI;
     int most = 0;
     for (int c : cloths) {
         const ClothSys& S = C->sys[c];
-        if (S.bandwidth > 32767) return false;
+        if (S.bandwidth > 32767) return p;
+        if (pre == PRE_AMG) {
+            const int bottom = dense ? S.amg.smallL0 : S.amg.nl - 1;
+            if (bottom >= MAXL || S.amg.L[bottom].n > BOTTOM) return p;
+        }
         local = local && S.nn <= 512;
         most = std::max(most, S.nn);
     }
+    // Large lone systems stream their factor or their coarse levels from memory either way (learned:
+    // 65,536 rows 11.0 against 13.6 ms a solve, 131,044 rows 23.8 against 20.0; multigrid: 90,000
+    // rows 7.8 against 8.7, 129,600 rows 10.4 against 9.8).
+    if ((pre == PRE_LEARNED && most > 65536) || (pre == PRE_AMG && most > 98304)) return p;
+    // more rows than the launches hold
+    long rows = 0;
+    for (int c : cloths) rows += 512l * cdiv(C->sys[c].nn, 512);
+    const int launches = pre == PRE_JACOBI ? 2 : 1;
+    if (rows > launches * 131072l) return p;
     // Rows per workgroup: one workgroup and LDS for systems of 512 rows; otherwise a lone system is
     // spread over more CUs by 256 (1,089 rows: 4.6 us an iteration with 256, 6.1 with 512), until the
     // meeting of many workgroups costs more (65,536 rows: 12.6 us with 256, 9.1 with 512).  A batch
     // fills the CUs anyway (32 cloths, 170,000 rows: 24.6 ms with 256, 15.9 with 512).
-    const int T = local || n > 1 || most > 96 * 256 ? 512 : 256;
-    const void* f = kernel_of(T, local);
-    const int cap = resident(C, f, T);
-    std::vector<int> G(n), order(n);
+    const int T = p.T = local || n > 1 || most > 96 * 256 ? 512 : 256;
+    p.f = kernel_of(T, local, pre);
+    const int cap = resident(C, p.f, T);
+    std::vector<int>& G = p.G;
+    std::vector<int> order(n);
+    G.resize(n);
     for (int k = 0; k < n; k++) {
-        G[k] = cdiv(C->sys[cloths[k]].nn, T);
+        const ClothSys& S = C->sys[cloths[k]];
+        G[k] = cdiv(S.nn, T);
+        if (pre == PRE_AMG && dense) {
+            // workgroups without rows join the group where the bottom's dense operator is more than
+            // 128 KB a workgroup (4,225 rows on 17 workgroups and an operator of 8.4 MB: 4.9 ms a
+            // solve, 3.5 with 72) or more than four rows a wave
+            const int dim = 3 * S.amg.L[S.amg.smallL0].n;
+            G[k] = std::max(G[k], std::max(cdiv((long)dim * dim * 4, 128 << 10), cdiv(dim, 4 * (T / 64))));
+        }
         order[k] = k;
-        if (((G[k] + 7) & ~7) > cap) return false;
+        if (((G[k] + 7) & ~7) > cap) return p;
     }
     // Launches of as many groups as fit, largest systems first (they iterate longest).  Workgroups are
     // dealt to the 8 XCDs round-robin; a group of a batch goes to the least loaded XCD, whose L2 its
@@ -538,9 +918,6 @@ bool ppcg_solve(cs_ctx* C, const std::vector<int>& cloths, int* iters, float* re
     // waits out its slowest system (340,000 rows in 48 cloths: 37.6 against 40 ms; 170,000 in 32:
     // 15.9 against 22.5).
     std::sort(order.begin(), order.end(), [&](int a, int b) { return G[a] != G[b] ? G[a] > G[b] : a < b; });
-    struct Round { int off, n; };
-    std::vector<Round> rounds;
-    std::vector<int2> map;
     for (size_t at = 0; at < order.size();) {
         std::vector<int2> xcd[8];
         size_t deep = 0;
@@ -565,11 +942,21 @@ bool ppcg_solve(cs_ctx* C, const std::vector<int>& cloths, int* iters, float* re
             }
             for (auto& v : xcd) deep = std::max(deep, v.size());
         }
-        rounds.push_back({(int)map.size(), (int)(8 * deep)});
+        p.rounds.push_back({(int)p.map.size(), (int)(8 * deep)});
         for (size_t d = 0; d < deep; d++)
-            for (int y = 0; y < 8; y++) map.push_back(d < xcd[y].size() ? xcd[y][d] : make_int2(-1, 0));
+            for (int y = 0; y < 8; y++) p.map.push_back(d < xcd[y].size() ? xcd[y][d] : make_int2(-1, 0));
     }
-    if (rounds.size() > 2) return false;
+    p.fits = (int)p.rounds.size() <= launches;
+    return p;
+}
+
+// Results per entry of `cloths`, as pcg_solve.  False, and nothing solved, when a launch is refused or a
+// group gives up.
+bool run_plan(cs_ctx* C, const Plan& p, const std::vector<int>& cloths, int pre, bool dense, int* iters, float* relres,
+              int* converged) {
+    const int n = (int)cloths.size(), T = p.T;
+    const std::vector<int>& G = p.G;
+    const std::vector<int2>& map = p.map;
     hipStream_t s = C->stream;
     std::vector<size_t> so(n);
     size_t words = 0;
@@ -580,7 +967,7 @@ bool ppcg_solve(cs_ctx* C, const std::vector<int>& cloths, int* iters, float* re
     uint64_t* slots = C->ppSlots.as<uint64_t>(words);
     PcgScalars* out = C->bScal.as<PcgScalars>(n);
     std::vector<PSys> tab(n);
-    for (int k = 0; k < n; k++) tab[k] = describe(C->sys[cloths[k]], G[k], slots + so[k], out + k);
+    for (int k = 0; k < n; k++) tab[k] = describe(C->sys[cloths[k]], pre, dense, G[k], slots + so[k], out + k);
     PSys* dtab = C->ppTab.as<PSys>(n);
     int2* dmap = C->ppMap.as<int2>(map.size());
     PcgScalars* h = static_cast<PcgScalars*>(pinned_batch(C, sizeof(PcgScalars) * n));
@@ -590,13 +977,13 @@ bool ppcg_solve(cs_ctx* C, const std::vector<int>& cloths, int* iters, float* re
     fill_u32(reinterpret_cast<uint32_t*>(out), 0u, (long)n * (sizeof(PcgScalars) / 4), s);
     float tol2 = C->P.pcg_rel_tol * C->P.pcg_rel_tol;
     int maxit = C->P.pcg_max_iters;
-    for (const Round& r : rounds) {
+    for (const Round& r : p.rounds) {
         const PSys* ct = dtab;
         const int2* cm = dmap + r.off;
         void* args[] = {(void*)&ct, (void*)&cm, (void*)&tol2, (void*)&maxit};
-        const hipError_t e = hipLaunchCooperativeKernel(f, dim3(r.n), dim3(T), args, 0, s);
+        const hipError_t e = hipLaunchCooperativeKernel(p.f, dim3(r.n), dim3(T), args, 0, s);
         if (e != hipSuccess) {
-            // too large, or another process holds the device's cooperative queue
+                // too large, or another process holds the device's cooperative queue
             (void)hipGetLastError();
             CS_HIP(hipStreamSynchronize(s));
             C->ppOff = true;
@@ -615,6 +1002,49 @@ bool ppcg_solve(cs_ctx* C, const std::vector<int>& cloths, int* iters, float* re
         relres[k] = h[k].bb > 0.0f ? sqrtf(h[k].rr / h[k].bb) : 0.0f;
         converged[k] = h[k].rr <= h[k].tol2bb;
         C->sys[cloths[k]].solved = converged[k] != 0;
+    }
+    return true;
+}
+
+bool allowed(const cs_ctx* C) {
+    return !C->ppOff && !(C->P.flags & (CS_FLAG_TIME_KERNELS | CS_FLAG_GRAPH_CYCLES));
+}
+
+}  // namespace
+
+bool ppcg_solve(cs_ctx* C, int c, bool amg, bool learned, int* iters, float* relres, int* converged) {
+    // the cycle with the learned smoother would meet 13 times an iteration: measured slower at every size
+    if (!allowed(C) || (amg && learned)) return false;
+    const int pre = amg ? PRE_AMG : learned ? PRE_LEARNED : PRE_JACOBI;
+    const std::vector<int> one{c};
+    const Plan p = plan_for(C, one, pre, true);
+    return p.fits && run_plan(C, p, one, pre, true, iters, relres, converged);
+}
+
+bool ppcg_solve_batch(cs_ctx* C, bool amg, int* iters, float* relres, int* converged) {
+    if (!allowed(C)) return false;
+    std::vector<int> part[2];  // block Jacobi, multigrid
+    const std::vector<int>* usable = amg ? &bamg_build(C) : nullptr;
+    for (int c = 0; c < C->nCloths; c++) part[usable && (*usable)[c] ? 1 : 0].push_back(c);
+    Plan plan[2];
+    for (int k = 0; k < 2; k++) {
+        if (part[k].empty()) continue;
+        plan[k] = plan_for(C, part[k], k ? PRE_AMG : PRE_JACOBI, false);
+        if (!plan[k].fits) return false;
+    }
+    if (amg) bamg_prepare(C);
+    for (int k = 0; k < 2; k++) {
+        if (part[k].empty()) continue;
+        const int n = (int)part[k].size();
+        std::vector<int> it(n), cv(n);
+        std::vector<float> rel(n);
+        if (!run_plan(C, plan[k], part[k], k ? PRE_AMG : PRE_JACOBI, false, it.data(), rel.data(), cv.data()))
+            return false;
+        for (int j = 0; j < n; j++) {
+            iters[part[k][j]] = it[j];
+            relres[part[k][j]] = rel[j];
+            converged[part[k][j]] = cv[j];
+        }
     }
     return true;
 }

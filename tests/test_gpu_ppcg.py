@@ -1,11 +1,12 @@
-"""Block-Jacobi PCG inside one launch (cs_ppcg.hip) against the separately launched iterations
+"""PCG inside one launch (cs_ppcg.hip) against the separately launched iterations
 (CS_FLAG_TIME_KERNELS keeps those), on the same assembled systems, at the sizes where the kernel's
 workgroups, registers and launches begin and end."""
 import numpy as np
 import pytest
 
 from clothsimulator_amd import CS_MESH_CLOTH, Simulator, scenes
-from clothsimulator_amd._cabi import (CS_FLAG_INSTANCES, CS_FLAG_TIME_KERNELS, MeshArrays, default_params,
+from clothsimulator_amd._cabi import (CS_FLAG_FIXED_TUNING, CS_FLAG_INSTANCES, CS_FLAG_TIME_KERNELS, CS_PRECOND_AMG,
+                                      CS_PRECOND_AMG_LEARNED, CS_PRECOND_LEARNED, MeshArrays, default_params,
                                       material_struct)
 
 pytestmark = pytest.mark.gpu
@@ -37,10 +38,10 @@ def _residual(system, dv):
     return np.linalg.norm(b - y.ravel()) / np.linalg.norm(b)
 
 
-def _compare(spec, x, v):
+def _compare(spec, x, v, **params):
     """The solve in one launch forms the same sums in the same order: the same bits."""
-    a, sa, system = _solve(spec, 0, x, v)
-    l, sl, _ = _solve(spec, CS_FLAG_TIME_KERNELS, x, v)
+    a, sa, system = _solve(spec, 0, x, v, **params)
+    l, sl, _ = _solve(spec, CS_FLAG_TIME_KERNELS, x, v, **params)
     assert sa.pcg_converged and sl.pcg_converged and sa.pcg_iters == sl.pcg_iters
     assert np.array_equal(a, l)
     # 1e-5 |b|, in FP64 up to the rounding of the assembled values that are read back (static and
@@ -54,6 +55,42 @@ def _compare(spec, x, v):
 def test_solve_equals_launched(n):
     spec = scenes.hang(n)
     _compare(spec, *_state(spec))
+
+
+# 9: the smallest hierarchy; 45, 46 and 156, 157 as above; 65: workgroups without rows share the
+# multigrid's dense operator; with the learned smoother only cloths without a hierarchy (8).
+@pytest.mark.parametrize("precond,n", [(CS_PRECOND_LEARNED, n) for n in (2, 16, 46, 157)] +
+                         [(CS_PRECOND_AMG, n) for n in (8, 9, 23, 45, 65, 129, 157)] +
+                         [(CS_PRECOND_AMG_LEARNED, n) for n in (8, 9, 33)])
+def test_preconditioned_solve_equals_launched(precond, n):
+    spec = scenes.crumple(n, height=0.01, sigma=0.05 / n)
+    x, v = _state(spec, amp=0.0)
+    _compare(spec, x, v, precond=precond)
+
+
+@pytest.mark.parametrize("precond", [CS_PRECOND_LEARNED, CS_PRECOND_AMG])
+def test_preconditioned_contacts_equal_launched(precond):
+    spec = scenes.fold(49, gap=9e-4, noise=5e-5)
+    x = spec.cloths[0].mesh.x
+    _compare(spec, x, np.zeros_like(x), precond=precond)
+
+
+def test_multigrid_batch_matches_launched():
+    """Sides 5 to 33 in one launch each for the cloths with and without a hierarchy, against the
+    launched batch; the coarsest levels are solved the same way."""
+    out = []
+    for flags in (0, CS_FLAG_TIME_KERNELS):
+        spec = scenes.instances(count=6, seed=3, side_lo=5, side_hi=33, gap=8e-4)
+        sides = sorted(int(round(np.sqrt(c.mesh.n_nodes))) for c in spec.cloths)
+        assert sides[0] <= 8 and sides[-1] > 22
+        spec.params.precond = CS_PRECOND_AMG
+        spec.params.flags |= flags | CS_FLAG_FIXED_TUNING
+        sim = Simulator(spec)
+        s, st = sim.physics_step()
+        assert s == 0 and st.pcg_rel_residual <= 1e-5
+        out.append((st.pcg_iters, [sim.state(CS_MESH_CLOTH, k)[0] for k in range(6)]))
+    assert abs(out[0][0] - out[1][0]) <= 6
+    assert max(np.abs(a - b).max() for a, b in zip(out[0][1], out[1][1])) <= 1e-5
 
 
 @pytest.mark.parametrize("n", [362, 363])

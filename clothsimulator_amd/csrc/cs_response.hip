@@ -10,8 +10,11 @@
 // The impact nodes are de-duplicated by a stable radix sort of (node, slot),
 // which also gives every node the list of its constraint slots in ascending
 // order, so gradients are gathered (no atomics).  The whole iteration, line
-// search included, runs in one 1024-thread workgroup: the reference's host
-// round trip per line-search evaluation is gone.
+// search included, runs in one workgroup: the reference's host round trip per
+// line-search evaluation is gone.  Up to LDS_SLOTS constraint slots the solve
+// stays in registers and LDS (k_opt_solve_lds); above, k_opt_solve reads its
+// operands from memory on every evaluation.  Both add in the same order and
+// give the same bits.
 #include "cs_kernels.hpp"
 #include "cs_math.hpp"
 
@@ -192,6 +195,195 @@ __global__ void __launch_bounds__(OB) k_opt_solve(OptArgs<View> A, int* iterOut)
     if (threadIdx.x == 0 && iterOut) *iterOut = iter;
 }
 
+// ---- the solve in registers and LDS ----------------------------------------
+// The solve is a serial chain of up to 100 gradient steps, each a few short sums over at most some
+// thousand nodes and constraints, so what bounds it is latency: in k_opt_solve every evaluation
+// walks slot -> node -> position through memory and spends three barriers per sum.  Here a thread
+// keeps its nodes (position, gradient, target, weight) and its constraint (normal, weights,
+// multiplier) in registers; positions, coefficients and the slot lists are in LDS.  The constraint
+// values and the objective of an accepted line-search point are those of the next evaluation, so
+// they are not computed again; two sums share one barrier.  A cloth of 129x129 nodes draped on a
+// sphere: 0.72 ms a call in k_opt_solve, 0.19 ms here (100 steps); 16 / 64 / 256 / 1024 random
+// impacts, 100 steps: 0.11 / 0.14 / 0.23 / 0.42 ms.
+constexpr int LDS_SLOTS = 4 * OB;
+constexpr int LDS_SMALL = 256;  // one slot per thread of four wavefronts
+
+template <int CTRL>
+__device__ __forceinline__ float dpp_add(float v) {
+    return v + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, false));
+}
+
+// The sum over a wavefront, in every lane.  The pairs are those of shuffles by 32, 16, 8, 4, 2, 1
+// (wg_sum): after the step by 8 a row holds equal values 8 lanes apart, so a rotation by 4 reads
+// the partner of the shuffle by 4, and so on down.
+__device__ __forceinline__ float wave_sum(float v) {
+    auto h = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = __uint_as_float(h[0]) + __uint_as_float(h[1]);
+    auto q = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = __uint_as_float(q[0]) + __uint_as_float(q[1]);
+    v = dpp_add<0x128>(v);  // row_ror:8
+    v = dpp_add<0x124>(v);
+    v = dpp_add<0x122>(v);
+    return dpp_add<0x121>(v);
+}
+
+// Sums of two values over the workgroup, in the order of wg_sum, with one barrier of its own; the
+// caller has another between two sums (part is read after the barrier).
+template <int T>
+__device__ __forceinline__ float2 wg_sum2(float a, float b, float2* part) {
+    a = wave_sum(a);
+    b = wave_sum(b);
+    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = make_float2(a, b);
+    __syncthreads();
+    float2 s = make_float2(0.0f, 0.0f);
+#pragma unroll
+    for (int w = 0; w < T / 64; w++) {
+        s.x += part[w].x;
+        s.y += part[w].y;
+    }
+    return s;
+}
+
+// LDS, in bytes per slot and constraint: 16 position, 8 (constraint, weight) in node order, 4 the
+// slot's position; 16 normal and coefficient.
+constexpr size_t lds_bytes(int K, int nC) { return (size_t)K * nC * 28 + (size_t)nC * 16; }
+
+// T threads of NU nodes each: K * nC <= T * NU (a node has a slot), nC <= T.
+template <class View, int T, int NU>
+__global__ void __launch_bounds__(T) k_opt_solve_lds(OptArgs<View> A, int* iterOut) {
+    constexpr int K = View::K;
+    extern __shared__ float4 mem[];
+    __shared__ float2 part[T / 64];
+    const int nN = (int)*A.nNptr;
+    if (nN == 0) return;
+    const int m = K * A.nC, t = threadIdx.x;
+    float4* pos = mem;                                  // [m]: node u at u, a fixed slot at its sorted place (>= nN)
+    float4* con = pos + m;                              // [nC]: normal, coefficient
+    float2* rec = reinterpret_cast<float2*>(con + A.nC);  // [m]: constraint (int bits), weight
+    int* at = reinterpret_cast<int*>(rec + m);          // [m]: where the slot's position is
+
+    for (int k = t; k < m; k += T) {
+        const int slot = (int)A.sortedSlots[k], i = slot / K, j = slot % K, u = A.slotMap[slot];
+        rec[k] = make_float2(__int_as_float(i), A.V.w(i, j));
+        at[slot] = u > -1 ? u : k;
+        if (u < 0) pos[k] = A.x[A.V.node(i, j)];
+    }
+    V3f X[NU], G[NU], X1[NU];
+    float mass[NU];
+    int first[NU], last[NU];
+    float im = 0.0f, a = 0.0f;
+#pragma unroll
+    for (int r = 0; r < NU; r++) {
+        const int u = t + r * T;
+        X[r] = G[r] = X1[r] = mk(0.0f, 0.0f, 0.0f);
+        mass[r] = 0.0f;
+        first[r] = last[r] = 0;
+        if (u < nN) {
+            const int nd = A.nodes[u];
+            X[r] = ld3(A.x[nd]);
+            X1[r] = ld3(A.x1[nd]);
+            mass[r] = nd < A.NC ? A.mass[nd] : A.obstacleMass;
+            first[r] = A.start[u];
+            last[r] = A.end[u];
+            pos[u] = st4(X[r]);
+            im += 1.0f / mass[r];
+            a += mass[r] * norm2(X[r] - X1[r]);
+        }
+    }
+    const float2 ia = wg_sum2<T>(im, a, part);
+    const float invMass = ia.x / (float)nN;
+    float obj = 0.5f * ia.y * invMass;
+    V3f n = mk(0.0f, 0.0f, 0.0f);
+    float w[K], lambda = 0.0f;
+    int p[K];
+    if (t < A.nC) {
+        n = A.V.n(t);
+#pragma unroll
+        for (int j = 0; j < K; j++) {
+            w[j] = A.V.w(t, j);
+            p[j] = at[K * t + j];
+        }
+    }
+    const float mu = 1e3f;
+    // c_t at the published positions
+    auto constraint_at = [&]() {
+        float c = -A.thickness;
+#pragma unroll
+        for (int j = 0; j < K; j++) c += w[j] * dot(n, ld3(pos[p[j]]));
+        return c;
+    };
+    auto penalty = [&](float coef) { return coef != 0.0f ? 0.5f * mu * (coef * coef) : 0.0f; };
+    // the objective's terms at X - s G
+    auto distance = [&](float s) {
+        float a = 0.0f;
+#pragma unroll
+        for (int r = 0; r < NU; r++)
+            if (t + r * T < nN) a += mass[r] * norm2((X[r] - s * G[r]) - X1[r]);
+        return a;
+    };
+    float c = t < A.nC ? constraint_at() : 0.0f;
+    float s = 1e-3f * (float)nN;
+    int iter = 0;
+    for (; iter < 100; iter++) {
+        // valueAndGradient (src/optimization/Optimization.cu:33-49)
+        float pen = 0.0f;
+        if (t < A.nC) {
+            const float coef = tmin(c + lambda / mu, 0.0f);
+            con[t] = make_float4(n.x, n.y, n.z, coef);
+            pen = penalty(coef);
+        }
+        __syncthreads();
+        float g2 = 0.0f;
+#pragma unroll
+        for (int r = 0; r < NU; r++) {
+            if (t + r * T >= nN) continue;
+            V3f g = (invMass * mass[r]) * (X[r] - X1[r]);
+            for (int k = first[r]; k < last[r]; k++) {
+                const float2 q = rec[k];
+                const float4 e = con[__float_as_int(q.x)];
+                if (e.w != 0.0f) g += ((mu * e.w) * q.y) * mk(e.x, e.y, e.z);
+            }
+            G[r] = g;
+            g2 += norm2(g);
+        }
+        const float2 pg = wg_sum2<T>(pen, g2, part);
+        const float f = obj + pg.x, norm2g = pg.y;
+        s /= 0.7f;
+        float ft, objt;
+        do {
+            s *= 0.7f;
+#pragma unroll
+            for (int r = 0; r < NU; r++)
+                if (t + r * T < nN) pos[t + r * T] = st4(X[r] - s * G[r]);
+            __syncthreads();
+            pen = 0.0f;
+            if (t < A.nC) {
+                c = constraint_at();
+                pen = penalty(tmin(c + lambda / mu, 0.0f));
+            }
+            const float2 op = wg_sum2<T>(distance(s), pen, part);
+            objt = 0.5f * op.x * invMass;
+            ft = objt + op.y;
+        } while (ft >= f - 0.5f * s * norm2g && s >= 1e-12f && tabs(f - ft) >= 1e-10f);
+        if (s < 1e-12f || tabs(f - ft) < 1e-10f) break;
+#pragma unroll
+        for (int r = 0; r < NU; r++)
+            if (t + r * T < nN) X[r] = X[r] - s * G[r];
+        obj = objt;
+        // updateMultiplier (src/optimization/Optimization.cu:51-57)
+        if (t < A.nC) lambda = tmin(lambda + mu * c, 0.0f);
+    }
+#pragma unroll
+    for (int r = 0; r < NU; r++)
+        if (t + r * T < nN) A.x[A.nodes[t + r * T]] = st4(X[r]);
+    if (t == 0 && iterOut) *iterOut = iter;
+}
+
+template <class View, int T, int NU>
+void launch_lds(const OptArgs<View>& A, int* iterOut, hipStream_t s) {
+    hipLaunchKernelGGL((k_opt_solve_lds<View, T, NU>), dim3(1), dim3(T), lds_bytes(View::K, A.nC), s, A, iterOut);
+}
+
 template <class View>
 void opt_response(cs_ctx* C, View V, int nImp, int deform, const float* weight, float obstacleWeight) {
     if (nImp <= 0) return;
@@ -235,7 +427,12 @@ void opt_response(cs_ctx* C, View V, int nImp, int deform, const float* weight, 
     A.lambda = C->optLambda.as<float>(nImp);
     A.coef = C->optCoef.as<float>(nImp);
     int* iterOut = C->optScal.as<int>(4);
-    hipLaunchKernelGGL(k_opt_solve<View>, dim3(1), dim3(OB), 0, s, A, iterOut);
+    // A slot per thread while the slots fit a workgroup of four or sixteen wavefronts (fewer waves
+    // make shorter barriers and sums), four up to LDS_SLOTS (LDS: 128 KiB then).
+    if (m <= LDS_SMALL) launch_lds<View, LDS_SMALL, 1>(A, iterOut, s);
+    else if (m <= OB) launch_lds<View, OB, 1>(A, iterOut, s);
+    else if (m <= LDS_SLOTS) launch_lds<View, OB, 4>(A, iterOut, s);
+    else hipLaunchKernelGGL(k_opt_solve<View>, dim3(1), dim3(OB), 0, s, A, iterOut);
     CS_LAUNCH_CHECK();
 }
 

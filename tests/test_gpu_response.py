@@ -18,7 +18,7 @@ import oracle
 from clothsimulator_amd import CS_MESH_CLOTH, CS_MESH_OBSTACLE, Simulator
 from clothsimulator_amd._cabi import CS_E_COLLISION_FAILED, CS_E_NOT_CONVERGED, CS_OK
 from clothsimulator_amd.scenes import fold, hang
-from test_oracle_response import response_scene, vf_impact
+from test_oracle_response import IMPACT_DTYPE, response_scene, vf_impact
 
 pytestmark = pytest.mark.gpu
 
@@ -114,3 +114,44 @@ def test_collision_failure_is_reported_not_fatal(iters):
     sim.set_params(p)
     s, _ = sim.collision_step()
     assert s == CS_OK
+
+
+@pytest.mark.parametrize("n", [1, 2, 63, 64, 65, 255, 256, 257, 700, 1024])
+def test_impact_response_sizes_agree_with_the_general_kernel(n):
+    """Calls of up to 1024 impacts (4096 slots) are solved in registers and LDS, in workgroups of
+    256 threads up to 64 impacts and of 1024 with one or four nodes a thread up to 256 and 1024;
+    larger ones read their operands from memory.  Impacts between obstacle nodes alone whose
+    constraint holds add no unknown and only zero terms, so the same impacts with such ones behind
+    them go to the general kernel and must give the same iterations and the same bits."""
+    spec = hang(41)
+    spec.obstacles.append(response_scene().obstacles[0])
+    sim = Simulator(spec)
+    x = _positions(sim)
+    nc = len(sim.state(CS_MESH_CLOTH, 0)[0])
+    rng = np.random.default_rng(n)
+    far = nc + int(np.argmax(np.linalg.norm(x[nc:], axis=1)))
+    imps = np.zeros(n, dtype=IMPACT_DTYPE)
+    for k in range(n):
+        nodes = rng.choice(nc, 4, replace=False)
+        if k % 5 == 0:
+            nodes[3] = far  # a fixed slot among free ones
+        b = rng.dirichlet(np.ones(3))
+        nrm = rng.standard_normal(3)
+        imps[k]["nodes"], imps[k]["w"] = nodes, [1.0, *-b]
+        imps[k]["n"] = nrm / np.linalg.norm(nrm)
+        gap = (imps[k]["w"][:, None] * x[nodes]).sum(axis=0) @ imps[k]["n"]
+        if gap > 0:  # mostly violated
+            imps[k]["n"] *= -1.0
+    pad = np.zeros(1025, dtype=imps.dtype)
+    pad["nodes"], pad["w"] = far, [1.0, 0.0, 0.0, 0.0]
+    pad["n"] = x[far] / np.linalg.norm(x[far])
+    res = []
+    for recs in (imps, np.concatenate([imps, pad])):
+        s = Simulator(spec)
+        it = s.impact_response(recs, 0)
+        res.append((it, _positions(s)))
+    moved = int((np.abs(res[0][1] - x).max(axis=1) > 0).sum())
+    print("%d impacts: %d and %d iterations, %d nodes moved" % (n, res[0][0], res[1][0], moved))
+    assert moved > n and np.isfinite(res[0][1]).all()
+    assert res[0][0] == res[1][0]
+    assert np.array_equal(res[0][1], res[1][1])

@@ -12,9 +12,8 @@
 // order, so gradients are gathered (no atomics).  The whole iteration, line
 // search included, runs in one workgroup: the reference's host round trip per
 // line-search evaluation is gone.  Up to LDS_SLOTS constraint slots the solve
-// stays in registers and LDS (k_opt_solve_lds); above, k_opt_solve reads its
-// operands from memory on every evaluation.  Both add in the same order and
-// give the same bits.
+// stays in registers and LDS (k_opt_solve_lds); above, k_opt_solve keeps
+// them in memory.  Both add in the same order and give the same bits.
 #include "cs_kernels.hpp"
 #include "cs_math.hpp"
 
@@ -70,20 +69,40 @@ __global__ void k_opt_map(int m, int N, const uint64_t* __restrict__ keys, const
     if (k + 1 == m || keys[k + 1] != key) end[u] = k + 1;
 }
 
-__device__ float wg_sum(float v, float* lds) {
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+template <int CTRL>
+__device__ __forceinline__ float dpp_add(float v) {
+    return v + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, false));
+}
+
+// The sum over a wavefront, in every lane.  The pairs are those of shuffles by 32, 16, 8, 4, 2, 1:
+// after the step by 8 a row holds equal values 8 lanes apart, so a rotation by 4 reads the partner
+// of the shuffle by 4, and so on down.
+__device__ __forceinline__ float wave_sum(float v) {
+    auto h = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = __uint_as_float(h[0]) + __uint_as_float(h[1]);
+    auto q = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = __uint_as_float(q[0]) + __uint_as_float(q[1]);
+    v = dpp_add<0x128>(v);  // row_ror:8
+    v = dpp_add<0x124>(v);
+    v = dpp_add<0x122>(v);
+    return dpp_add<0x121>(v);
+}
+
+// Sums of two values over the workgroup (the wavefronts in order) with one barrier of its own; the
+// caller has another between two sums (part is read after the barrier).
+template <int T>
+__device__ __forceinline__ float2 wg_sum2(float a, float b, float2* part) {
+    a = wave_sum(a);
+    b = wave_sum(b);
+    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = make_float2(a, b);
+    __syncthreads();
+    float2 s = make_float2(0.0f, 0.0f);
 #pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-    __syncthreads();
-    if (lane == 0) lds[wave] = v;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        float s = 0.0f;
-        for (int w = 0; w < OB / 64; w++) s += lds[w];
-        lds[OB / 64] = s;
+    for (int w = 0; w < T / 64; w++) {
+        s.x += part[w].x;
+        s.y += part[w].y;
     }
-    __syncthreads();
-    return lds[OB / 64];
+    return s;
 }
 
 template <class View>
@@ -101,148 +120,139 @@ struct OptArgs {
     const float* mass;  // per node: the objective's weight (mass for impacts, area for separation)
     int NC;
     float obstacleMass, thickness;  // obstacle nodes' weight
-    float4 *X, *Xn, *G;
-    float *lambda, *coef;
+    // k_opt_solve's working set.  Per node: position, gradient, target and weight.  pos: node u's
+    // trial position at u, a fixed slot's at its sorted place.  con: normal and coefficient.
+    // rec, in node order: a slot's constraint (int bits) and weight; slot, by slot: where its
+    // position is (int bits) and its weight.
+    float4 *X, *G, *X1, *pos, *con;
+    float2 *rec, *slot;
+    float *lambda, *c;
 };
 
-template <class View>
-__device__ __forceinline__ float node_mass(const OptArgs<View>& A, int u) {
-    int nd = A.nodes[u];
-    return nd < A.NC ? A.mass[nd] : A.obstacleMass;
-}
-
-template <class View>
-__device__ float constraint(const OptArgs<View>& A, const float4* Xp, int i) {
-    const V3f n = A.V.n(i);
-    float c = -A.thickness;
-    for (int j = 0; j < View::K; j++) {
-        int u = A.slotMap[View::K * i + j];
-        V3f p = u > -1 ? ld3(Xp[u]) : ld3(A.x[A.V.node(i, j)]);
-        c += A.V.w(i, j) * dot(n, p);
-    }
-    return c;
-}
-
-// value(x) (src/optimization/Optimization.cu:20-31): objective + penalty terms
-template <class View>
-__device__ float value(const OptArgs<View>& A, int nN, const float4* Xp, float invMass, float mu, float* lds,
-                       bool storeCoef) {
-    float a = 0.0f;
-    for (int u = threadIdx.x; u < nN; u += OB) {
-        V3f d = ld3(Xp[u]) - ld3(A.x1[A.nodes[u]]);
-        a += node_mass(A, u) * norm2(d);
-    }
-    float obj = 0.5f * wg_sum(a, lds) * invMass;
-    float pen = 0.0f;
-    for (int i = threadIdx.x; i < A.nC; i += OB) {
-        float coef = tmin(constraint(A, Xp, i) + A.lambda[i] / mu, 0.0f);
-        if (storeCoef) A.coef[i] = coef;
-        if (coef != 0.0f) pen += 0.5f * mu * (coef * coef);
-    }
-    return obj + wg_sum(pen, lds);
-}
-
-template <class View>
+// The solve of any size: thread t owns the nodes and constraints t, t + OB, ...  What it reads per
+// evaluation is gathered once into short FP32 records; the constraint values and the objective of an
+// accepted line-search point are those of the next evaluation and are not computed again.  Bound by
+// the latency of slot -> position: positions and coefficients are in LDS while they fit (1,025 random
+// impacts, 100 steps: 0.97 ms with them in memory, 0.64 in LDS; 2,000: 0.87; 2,023, in memory: 1.43).
+template <class View, bool LDS>
 __global__ void __launch_bounds__(OB) k_opt_solve(OptArgs<View> A, int* iterOut) {
-    __shared__ float lds[OB / 64 + 1];
+    constexpr int K = View::K;
+    extern __shared__ float4 mem[];
+    __shared__ float2 part[OB / 64];
     const int nN = (int)*A.nNptr;
     if (nN == 0) return;
-    float im = 0.0f;
-    for (int u = threadIdx.x; u < nN; u += OB) im += 1.0f / node_mass(A, u);
-    const float invMass = wg_sum(im, lds) / (float)nN;
-    for (int u = threadIdx.x; u < nN; u += OB) A.X[u] = A.x[A.nodes[u]];
-    for (int i = threadIdx.x; i < A.nC; i += OB) A.lambda[i] = 0.0f;
-    __syncthreads();
+    const int m = K * A.nC, t = threadIdx.x;
+    float4 *pos, *con;
+    if constexpr (LDS) { pos = mem; con = mem + m; }
+    else { pos = A.pos; con = A.con; }
+    for (int k = t; k < m; k += OB) {
+        const int slot = (int)A.sortedSlots[k], i = slot / K, j = slot % K, u = A.slotMap[slot];
+        const float w = A.V.w(i, j);
+        A.rec[k] = make_float2(__int_as_float(i), w);
+        A.slot[slot] = make_float2(__int_as_float(u > -1 ? u : k), w);
+        if (u < 0) pos[k] = A.x[A.V.node(i, j)];
+    }
+    float im = 0.0f, a = 0.0f;
+    for (int u = t; u < nN; u += OB) {
+        const int nd = A.nodes[u];
+        const V3f x = ld3(A.x[nd]), x1 = ld3(A.x1[nd]);
+        const float mass = nd < A.NC ? A.mass[nd] : A.obstacleMass;
+        A.X[u] = pos[u] = st4(x);
+        A.X1[u] = st4(x1, mass);
+        im += 1.0f / mass;
+        a += mass * norm2(x - x1);
+    }
+    const float2 ia = wg_sum2<OB>(im, a, part);
+    const float invMass = ia.x / (float)nN;
+    float obj = 0.5f * ia.y * invMass;
     const float mu = 1e3f;
+    // c_i at the published positions
+    auto constraint_at = [&](int i, V3f n) {
+        float c = -A.thickness;
+#pragma unroll
+        for (int j = 0; j < K; j++) {
+            const float2 q = A.slot[K * i + j];
+            c += q.y * dot(n, ld3(pos[__float_as_int(q.x)]));
+        }
+        return c;
+    };
+    auto penalty = [&](float coef) { return coef != 0.0f ? 0.5f * mu * (coef * coef) : 0.0f; };
+    for (int i = t; i < A.nC; i += OB) {
+        const V3f n = A.V.n(i);
+        con[i] = st4(n);
+        A.lambda[i] = 0.0f;
+        A.c[i] = constraint_at(i, n);
+    }
     float s = 1e-3f * (float)nN;
     int iter = 0;
     for (; iter < 100; iter++) {
         // valueAndGradient (src/optimization/Optimization.cu:33-49)
-        const float f = value(A, nN, A.X, invMass, mu, lds, true);
+        float pen = 0.0f;
+        for (int i = t; i < A.nC; i += OB) {
+            const float coef = tmin(A.c[i] + A.lambda[i] / mu, 0.0f);
+            con[i].w = coef;
+            pen += penalty(coef);
+        }
         __syncthreads();
         float g2 = 0.0f;
-        for (int u = threadIdx.x; u < nN; u += OB) {
-            V3f g = (invMass * node_mass(A, u)) * (ld3(A.X[u]) - ld3(A.x1[A.nodes[u]]));
-            for (int k = A.start[u]; k < A.end[u]; k++) {
-                const int slot = (int)A.sortedSlots[k];
-                const int i = slot / View::K, j = slot % View::K;
-                const float coef = A.coef[i];
-                if (coef != 0.0f) g += ((mu * coef) * A.V.w(i, j)) * A.V.n(i);
+        for (int u = t; u < nN; u += OB) {
+            const float4 x1 = A.X1[u];
+            V3f g = (invMass * x1.w) * (ld3(A.X[u]) - ld3(x1));
+            const int last = A.end[u];
+            float2 next = A.rec[A.start[u]];
+            for (int k = A.start[u]; k < last; k++) {
+                const float2 q = next;
+                next = A.rec[tmin(k + 1, m - 1)];
+                const float4 e = con[__float_as_int(q.x)];
+                if (e.w != 0.0f) g += ((mu * e.w) * q.y) * ld3(e);
             }
             A.G[u] = st4(g);
             g2 += norm2(g);
         }
-        const float norm2g = wg_sum(g2, lds);
+        const float2 pg = wg_sum2<OB>(pen, g2, part);
+        const float f = obj + pg.x, norm2g = pg.y;
         s /= 0.7f;
-        float ft;
+        float ft, objt;
         do {
             s *= 0.7f;
-            for (int u = threadIdx.x; u < nN; u += OB) A.Xn[u] = st4(ld3(A.X[u]) - s * ld3(A.G[u]));
+            a = 0.0f;
+            for (int u = t; u < nN; u += OB) {
+                const V3f x = ld3(A.X[u]) - s * ld3(A.G[u]);
+                const float4 x1 = A.X1[u];
+                pos[u] = st4(x);
+                a += x1.w * norm2(x - ld3(x1));
+            }
             __syncthreads();
-            ft = value(A, nN, A.Xn, invMass, mu, lds, false);
+            pen = 0.0f;
+            for (int i = t; i < A.nC; i += OB) {
+                const float c = constraint_at(i, ld3(con[i]));
+                A.c[i] = c;
+                pen += penalty(tmin(c + A.lambda[i] / mu, 0.0f));
+            }
+            const float2 op = wg_sum2<OB>(a, pen, part);
+            objt = 0.5f * op.x * invMass;
+            ft = objt + op.y;
         } while (ft >= f - 0.5f * s * norm2g && s >= 1e-12f && tabs(f - ft) >= 1e-10f);
         if (s < 1e-12f || tabs(f - ft) < 1e-10f) break;
-        for (int u = threadIdx.x; u < nN; u += OB) A.X[u] = A.Xn[u];
-        __syncthreads();
+        for (int u = t; u < nN; u += OB) A.X[u] = pos[u];
+        obj = objt;
         // updateMultiplier (src/optimization/Optimization.cu:51-57)
-        for (int i = threadIdx.x; i < A.nC; i += OB) A.lambda[i] = tmin(A.lambda[i] + mu * constraint(A, A.X, i), 0.0f);
-        __syncthreads();
+        for (int i = t; i < A.nC; i += OB) A.lambda[i] = tmin(A.lambda[i] + mu * A.c[i], 0.0f);
     }
-    for (int u = threadIdx.x; u < nN; u += OB) {
-        float4 p = A.X[u];
-        A.x[A.nodes[u]] = make_float4(p.x, p.y, p.z, 0.0f);
-    }
-    if (threadIdx.x == 0 && iterOut) *iterOut = iter;
+    for (int u = t; u < nN; u += OB) A.x[A.nodes[u]] = A.X[u];
+    if (t == 0 && iterOut) *iterOut = iter;
 }
 
 // ---- the solve in registers and LDS ----------------------------------------
 // The solve is a serial chain of up to 100 gradient steps, each a few short sums over at most some
-// thousand nodes and constraints, so what bounds it is latency: in k_opt_solve every evaluation
-// walks slot -> node -> position through memory and spends three barriers per sum.  Here a thread
-// keeps its nodes (position, gradient, target, weight) and its constraint (normal, weights,
-// multiplier) in registers; positions, coefficients and the slot lists are in LDS.  The constraint
-// values and the objective of an accepted line-search point are those of the next evaluation, so
-// they are not computed again; two sums share one barrier.  A cloth of 129x129 nodes draped on a
-// sphere: 0.72 ms a call in k_opt_solve, 0.19 ms here (100 steps); 16 / 64 / 256 / 1024 random
-// impacts, 100 steps: 0.11 / 0.14 / 0.23 / 0.42 ms.
+// thousand nodes and constraints, so latency bounds it.  Here a thread keeps its nodes (position,
+// gradient, target, weight) and its constraint (normal, weights, multiplier) in registers;
+// positions, coefficients and the slot lists are in LDS.  A cloth of 129x129 nodes draped on a
+// sphere: 0.72 ms a call with every operand in memory and three barriers per sum, 0.19 ms here (100
+// steps); 16 / 64 / 256 / 1024 random impacts, 100 steps: 0.11 / 0.14 / 0.23 / 0.42 ms.
 constexpr int LDS_SLOTS = 4 * OB;
 constexpr int LDS_SMALL = 256;  // one slot per thread of four wavefronts
-
-template <int CTRL>
-__device__ __forceinline__ float dpp_add(float v) {
-    return v + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, false));
-}
-
-// The sum over a wavefront, in every lane.  The pairs are those of shuffles by 32, 16, 8, 4, 2, 1
-// (wg_sum): after the step by 8 a row holds equal values 8 lanes apart, so a rotation by 4 reads
-// the partner of the shuffle by 4, and so on down.
-__device__ __forceinline__ float wave_sum(float v) {
-    auto h = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-    v = __uint_as_float(h[0]) + __uint_as_float(h[1]);
-    auto q = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-    v = __uint_as_float(q[0]) + __uint_as_float(q[1]);
-    v = dpp_add<0x128>(v);  // row_ror:8
-    v = dpp_add<0x124>(v);
-    v = dpp_add<0x122>(v);
-    return dpp_add<0x121>(v);
-}
-
-// Sums of two values over the workgroup, in the order of wg_sum, with one barrier of its own; the
-// caller has another between two sums (part is read after the barrier).
-template <int T>
-__device__ __forceinline__ float2 wg_sum2(float a, float b, float2* part) {
-    a = wave_sum(a);
-    b = wave_sum(b);
-    if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = make_float2(a, b);
-    __syncthreads();
-    float2 s = make_float2(0.0f, 0.0f);
-#pragma unroll
-    for (int w = 0; w < T / 64; w++) {
-        s.x += part[w].x;
-        s.y += part[w].y;
-    }
-    return s;
-}
+constexpr size_t LDS_POS_BYTES = 158 * 1024;  // of 160 KiB
 
 // LDS, in bytes per slot and constraint: 16 position, 8 (constraint, weight) in node order, 4 the
 // slot's position; 16 normal and coefficient.
@@ -412,7 +422,7 @@ void opt_response(cs_ctx* C, View V, int nImp, int deform, const float* weight, 
     hipLaunchKernelGGL(k_opt_map, dim3(cdiv(m, 256)), dim3(256), 0, s, m, C->N, keys, vals, flag, pos, nodes, start,
                        end, slotMap);
     CS_LAUNCH_CHECK();
-    OptArgs<View> A;
+    OptArgs<View> A{};
     A.nC = nImp;
     A.nNptr = pos + m;
     A.V = V;
@@ -421,18 +431,29 @@ void opt_response(cs_ctx* C, View V, int nImp, int deform, const float* weight, 
     A.NC = C->NC;
     A.obstacleMass = obstacleWeight;
     A.thickness = C->P.collision_thickness;
-    A.X = C->optX.as<float4>(m);
-    A.Xn = C->optNext.as<float4>(m);
-    A.G = C->optGrad.as<float4>(m);
-    A.lambda = C->optLambda.as<float>(nImp);
-    A.coef = C->optCoef.as<float>(nImp);
+    const size_t posBytes = sizeof(float4) * ((size_t)m + nImp);
+    const bool ldsPos = posBytes <= LDS_POS_BYTES;
+    if (m > LDS_SLOTS) {
+        A.X = C->optX.as<float4>(2 * (size_t)m);
+        A.X1 = A.X + m;
+        if (!ldsPos) {
+            A.pos = C->optNext.as<float4>(m);
+            A.con = C->optCoef.as<float4>(nImp);
+        }
+        A.rec = reinterpret_cast<float2*>(C->optGrad.as<float4>(2 * (size_t)m));
+        A.slot = A.rec + m;
+        A.G = reinterpret_cast<float4*>(A.slot + m);
+        A.lambda = C->optLambda.as<float>(2 * (size_t)nImp);
+        A.c = A.lambda + nImp;
+    }
     int* iterOut = C->optScal.as<int>(4);
     // A slot per thread while the slots fit a workgroup of four or sixteen wavefronts (fewer waves
     // make shorter barriers and sums), four up to LDS_SLOTS (LDS: 128 KiB then).
     if (m <= LDS_SMALL) launch_lds<View, LDS_SMALL, 1>(A, iterOut, s);
     else if (m <= OB) launch_lds<View, OB, 1>(A, iterOut, s);
     else if (m <= LDS_SLOTS) launch_lds<View, OB, 4>(A, iterOut, s);
-    else hipLaunchKernelGGL(k_opt_solve<View>, dim3(1), dim3(OB), 0, s, A, iterOut);
+    else if (ldsPos) hipLaunchKernelGGL((k_opt_solve<View, true>), dim3(1), dim3(OB), posBytes, s, A, iterOut);
+    else hipLaunchKernelGGL((k_opt_solve<View, false>), dim3(1), dim3(OB), 0, s, A, iterOut);
     CS_LAUNCH_CHECK();
 }
 

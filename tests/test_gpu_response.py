@@ -116,14 +116,14 @@ def test_collision_failure_is_reported_not_fatal(iters):
     assert s == CS_OK
 
 
-@pytest.mark.parametrize("n", [1, 2, 63, 64, 65, 255, 256, 257, 700, 1024])
+@pytest.mark.parametrize("n", [1, 2, 63, 64, 65, 255, 256, 257, 700, 1024, 1025, 2022])
 def test_impact_response_sizes_agree_with_the_general_kernel(n):
     """Calls of up to 1024 impacts (4096 slots) are solved in registers and LDS, in workgroups of
     256 threads up to 64 impacts and of 1024 with one or four nodes a thread up to 256 and 1024;
-    larger ones read their operands from memory.  Impacts between obstacle nodes alone whose
+    up to 2022 impacts the positions are in LDS, for more in memory.  Impacts between obstacle nodes alone whose
     constraint holds add no unknown and only zero terms, so the same impacts with such ones behind
     them go to the general kernel and must give the same iterations and the same bits."""
-    spec = hang(41)
+    spec = hang(65)
     spec.obstacles.append(response_scene().obstacles[0])
     sim = Simulator(spec)
     x = _positions(sim)
@@ -142,7 +142,7 @@ def test_impact_response_sizes_agree_with_the_general_kernel(n):
         gap = (imps[k]["w"][:, None] * x[nodes]).sum(axis=0) @ imps[k]["n"]
         if gap > 0:  # mostly violated
             imps[k]["n"] *= -1.0
-    pad = np.zeros(1025, dtype=imps.dtype)
+    pad = np.zeros(2023, dtype=imps.dtype)
     pad["nodes"], pad["w"] = far, [1.0, 0.0, 0.0, 0.0]
     pad["n"] = x[far] / np.linalg.norm(x[far])
     res = []

@@ -28,10 +28,10 @@
 // meeting per phase (restriction, pre-smoothing with residual, post-smoothing) instead of a launch.
 //
 // Measured (block Jacobi, solve time per iteration, separate launches -> here): 289 rows 14.1 -> 2.8 us,
-// 1,089 rows 13.5 -> 4.6, 16,641 rows with contacts 13.6 -> 7.9, 32,761 rows 13.9 -> 7.1,
+// 1,089 rows 13.5 -> 4.6, 16,641 rows with contacts 13.4 -> 7.5, 32,761 rows 13.9 -> 7.1,
 // 65,536 rows 18.0 -> 9.1, 129,600 rows 21.6 -> 15.3.
 // Solves with their set-up: learned factor 1,089 rows 3.9 -> 2.6 ms, 16,384 rows 9.0 -> 7.8, 32,400 rows
-// 9.5 -> 6.6; multigrid 289 rows 1.2 -> 0.8 ms, 4,225 rows 4.3 -> 3.6, 16,641 rows in contact 7.2 -> 5.8,
+// 9.5 -> 6.6; multigrid 289 rows 1.2 -> 0.8 ms, 4,225 rows 4.3 -> 3.7, 16,641 rows in contact 7.1 -> 5.4,
 // 32,400 rows 5.1 -> 3.6, 65,536 rows 7.4 -> 5.9.
 #include <algorithm>
 #include <cfloat>
@@ -366,6 +366,23 @@ __device__ __forceinline__ V3f postsmoothed(int i, const G1<int>* rp, const G1<i
 struct Pair {
     V3f z, d;
 };
+// a block's products with them, as floats of the products' LDS array and back
+__device__ __forceinline__ V3f times(const float (&o)[9], V3f v) { return mul3(o, v); }
+__device__ __forceinline__ Pair times(const float (&o)[9], Pair w) { return Pair{mul3(o, w.z), mul3(o, w.d)}; }
+__device__ __forceinline__ void toLds(float* p, V3f v) {
+    p[0] = v.x;
+    p[1] = v.y;
+    p[2] = v.z;
+}
+__device__ __forceinline__ void toLds(float* p, Pair w) {
+    toLds(p, w.z);
+    toLds(p + 3, w.d);
+}
+__device__ __forceinline__ void fromLds(const float* p, V3f& v) { v = mk(p[0], p[1], p[2]); }
+__device__ __forceinline__ void fromLds(const float* p, Pair& w) {
+    fromLds(p, w.z);
+    fromLds(p + 3, w.d);
+}
 // One row per thread, T rows per workgroup, one 64-row slice per wave; RS slots of a row in
 // registers (interior rows of a grid have 13), any further ones read from memory every iteration;
 // the gathers of GR slots are in flight together.  LOCAL: the system has one workgroup, whose
@@ -373,9 +390,10 @@ struct Pair {
 template <int T, int RS, int GR, bool LOCAL, int PRE>
 __global__ void __launch_bounds__(T, 2)  // 256 registers: the runtime refuses cooperative kernels of more
     k_ppcg(const PSys* __restrict__ tab, const int2* __restrict__ map, float tol2, int maxit) {
-    constexpr int NW = T / 64, CN = 2;
+    constexpr int NW = T / 64, CN = 3, CAP = LOCAL ? 2048 : 5120;
     __shared__ float red[2 * (NW + 4)];
     __shared__ int gaveUp;
+    __shared__ float prod[6 * CAP];  // products of contact blocks
     __shared__ float4 zl[LOCAL ? T : 1], dl[LOCAL ? T : 1];
     constexpr bool NET = PRE == PRE_LEARNED;
     __shared__ float lb[PRE == PRE_AMG ? 3 * BOTTOM : 1];  // the bottom level's right-hand side
@@ -430,22 +448,64 @@ __global__ void __launch_bounds__(T, 2)  // 256 registers: the runtime refuses c
     auto row = [&]() { return opaque(ic); };
     auto zAt = [&](int j) { return LOCAL ? v3(zl[j]) : v3(at((const G1<f3n>*)S.z, 16u * j)); };
     auto dAt = [&](const G1<f4n>* dp, int j) { return LOCAL ? v3(dl[j]) : v3(at((const G1<f3n>*)dp, 16u * j)); };
-    // The operand of a product is formed as it is gathered, gat(column); put(block, operand) adds.
-    auto contacts = [&](auto& gat, auto& put) {
+    // The operand of a product is formed as it is gathered, gat(column); put(block, operand) adds it to
+    // the row, add(product) adds a product.  A row's contacts, one thread and two blocks at a time:
+    auto contactsOfRow = [&](auto& gat, auto& put) {
         if (!S.contacts || !live) return;
         const int c1 = at(S.cRowPtr, 4u * row() + 4u);
-        for (int k = at(S.cRowPtr, 4u * row()); k < c1; k += CN) {  // CN blocks' loads in flight
-            float o[CN][9];
-            decltype(gat(0)) w[CN];
+        for (int k = at(S.cRowPtr, 4u * row()); k < c1; k += 2) {
+            float o[2][9];
+            decltype(gat(0)) w[2];
 #pragma unroll
-            for (int u = 0; u < CN; u++) {
+            for (int u = 0; u < 2; u++) {
                 const int kk = min(k + u, c1 - 1);
                 ldblk(S.cVal, kk, o[u]);
                 w[u] = gat(at(S.cCol, 4u * kk));
             }
 #pragma unroll
-            for (int u = 0; u < CN; u++)
+            for (int u = 0; u < 2; u++)
                 if (k + u < c1) put(o[u], w[u]);
+        }
+    };
+    // The contact blocks of the workgroup's rows: a row has none or dozens, and a thread that walks its
+    // own holds up its wave, so the threads share the blocks evenly, CN in flight each and neighbours in
+    // the matrix side by side, and a row's thread adds its products from LDS in order.  Solves, each row
+    // walked by its thread -> shared: 129x129 drape block Jacobi 8.6 -> 7.9 ms, multigrid 5.7 -> 5.4;
+    // 201x201 fold learned 19.7 -> 17.6 (18.9 with 2,048 products of LDS); few contacts: the same.
+    const int e0 = S.contacts ? S.cRowPtr[min(wg * T, nn)] : 0, e1 = S.contacts ? S.cRowPtr[min(wg * T + T, nn)] : 0;
+    auto contacts = [&](auto& gat, auto&& add) {
+        using W = decltype(gat(0));
+        constexpr int WF = sizeof(W) / sizeof(float);
+        if (e0 == e1) return;
+        const int r0 = at(S.cRowPtr, 4u * row()), r1 = at(S.cRowPtr, 4u * row() + 4u);
+        for (int base = e0; base < e1; base += CAP) {
+            const int end = min(base + CAP, e1);
+            if (base > e0) __syncthreads();
+            for (int k = base + tid; k < end; k += CN * T) {
+                float o[CN][9];
+                W w[CN];
+#pragma unroll
+                for (int u = 0; u < CN; u++) {
+                    const int kk = min(k + u * T, end - 1);
+                    ldblk(S.cVal, kk, o[u]);
+                    w[u] = gat(at(S.cCol, 4u * kk));
+                }
+#pragma unroll
+                for (int u = 0; u < CN; u++)
+                    if (k + u * T < end) toLds(prod + WF * (k + u * T - base), times(o[u], w[u]));
+            }
+            __syncthreads();
+            if (live) {
+                const int k1 = min(r1, end);
+                for (int k = max(r0, base); k < k1; k += 4) {
+                    W v[4];
+#pragma unroll
+                    for (int u = 0; u < 4; u++) fromLds(prod + WF * (min(k + u, k1 - 1) - base), v[u]);
+#pragma unroll
+                    for (int u = 0; u < 4; u++)
+                        if (k + u < k1) add(v[u]);
+                }
+            }
         }
     };
     // slots k0.. of the row from memory
@@ -460,7 +520,7 @@ __global__ void __launch_bounds__(T, 2)  // 256 registers: the runtime refuses c
         }
     };
     // the pattern's slots in order, then the contacts
-    auto sweep = [&](auto& gat, auto& put) {
+    auto sweep = [&](auto& gat, auto& put, auto&& add) {
         const int q = row();
 #pragma unroll
         for (int k = 0; k < (RS + 1) / 2; k++) asm volatile("" : "+v"(rel[k]));  // columns unpacked here, not kept
@@ -476,7 +536,7 @@ __global__ void __launch_bounds__(T, 2)  // 256 registers: the runtime refuses c
                 if (k0 + u < RS) put(a[k0 + u], w[u]);
         }
         streamed(RS, gat, put);
-        contacts(gat, put);
+        contacts(gat, add);
     };
     auto putZ = [&](V3f v) {
         if (LOCAL) zl[tid] = st4(v);
@@ -571,7 +631,7 @@ __global__ void __launch_bounds__(T, 2)  // 256 registers: the runtime refuses c
             V3f t = zero;
             auto gat = [&](int j) { return zAt(j); };
             auto put = [&](const float (&o)[9], V3f v) { acc3(t, o, v); };
-            sweep(gat, put);
+            sweep(gat, put, [&](V3f v) { t = t + v; });
             t = r - t;
             if (live) put3f(&at(gview(P.L[0]).t, 12u * row()), t);
             none[0] = 0.0f;
@@ -660,11 +720,10 @@ __global__ void __launch_bounds__(T, 2)  // 256 registers: the runtime refuses c
                     for (int c = 0; c < 9; c++) o[c] = at(av, 4u * ((k * 9 + c) * SLICE + lane));
                     acc3(y, o, ld3v(&at(e, 12u * at(ac, 4u * (k * SLICE + lane))), 0));
                 }
-                auto gatE = [&](int j) { return ld3v(&at(e, 12u * at(L.agg, 4u * j)), 0); };
-                auto putE = [&](const float (&o)[9], V3f v) { acc3(y, o, v); };
-                contacts(gatE, putE);
                 xs = xs + ld3v(&at(e, 12u * at(L.agg, 4u * row())), 0);
             }
+            auto gatE = [&](int j) { return ld3v(&at(e, 12u * at(L.agg, 4u * j)), 0); };
+            contacts(gatE, [&](V3f v) { y = y + v; });
             y = t - y;
             ldblk(S.Minv, row(), m);
             const V3f my = mul3(m, y);
@@ -689,7 +748,7 @@ __global__ void __launch_bounds__(T, 2)  // 256 registers: the runtime refuses c
             if (it == first) {
                 auto gat = [&](int j) { return zAt(j); };
                 auto put = [&](const float (&o)[9], V3f w) { acc3(q, o, w); };
-                sweep(gat, put);
+                sweep(gat, put, [&](V3f v) { q = q + v; });
                 d = z;
             } else {
                 const float beta = rz / rzOld;
@@ -700,7 +759,10 @@ __global__ void __launch_bounds__(T, 2)  // 256 registers: the runtime refuses c
                     acc3(q, o, w.z);
                     acc3(t, o, w.d);
                 };
-                sweep(gat, put);
+                sweep(gat, put, [&](Pair v) {
+                    q = q + v.z;
+                    t = t + v.d;
+                });
                 d = mk(z.x + beta * d.x, z.y + beta * d.y, z.z + beta * d.z);
                 q = mk(q.x + beta * t.x, q.y + beta * t.y, q.z + beta * t.z);
             }
@@ -734,7 +796,7 @@ __global__ void __launch_bounds__(T, 2)  // 256 registers: the runtime refuses c
                 y2 += (double)o[6] * xj.x + (double)o[7] * xj.y + (double)o[8] * xj.z;
             };
             streamed(0, zAt, put);
-            contacts(zAt, put);
+            contactsOfRow(zAt, put);
             const V3f b = ld3v(&at(S.b, 12u * row()), 0), bc = ld3v(&at(S.bc, 12u * row()), 0);
             r = mk((float)((double)b.x + (double)bc.x - y0), (float)((double)b.y + (double)bc.y - y1),
                    (float)((double)b.z + (double)bc.z - y2));

@@ -53,8 +53,7 @@ struct Bvh {
     int mesh = -1;
     int nf = 0;
     bool ccd = false;
-    DBuf keys, keysTmp;    // uint64 (morton) keys
-    DBuf vals, valsTmp;    // uint32 local face ids
+    DBuf keys;             // uint64 code<<32 | local face of the sorted leaves
     DBuf nodes;            // BNode[2nf-1]
     DBuf child;            // int2[nf-1]
     DBuf range;            // int2[nf-1]: first and last sorted leaf under each internal node

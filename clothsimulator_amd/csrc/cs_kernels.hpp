@@ -93,10 +93,8 @@ Xf motion_now(const cs_ctx* C, int motion);  // a motion at the context's curren
 void motion_place(cs_ctx* C);               // moving obstacles to x = x0 = T(now)(base)
 
 // LBVH (cs_lbvh.hip)
-void bvh_build(cs_ctx* C, int mesh, bool ccd);
-void bvh_build_all(cs_ctx* C, bool ccd);  // every mesh; small meshes in one batched launch
-void bvh_refit(cs_ctx* C, int mesh);
-void bvh_refit_range(cs_ctx* C, int m0, int m1);  // meshes [m0, m1); small meshes in one batched launch
+void bvh_build_all(cs_ctx* C, bool ccd);  // every mesh
+void bvh_refit_range(cs_ctx* C, int m0, int m1);  // meshes [m0, m1)
 // Candidate face pairs of all traversals (cloth self, cloth x earlier cloth,
 // cloth x obstacle) appended to C->pairs; returns the count.
 long bvh_all_pairs(cs_ctx* C, float thickness);

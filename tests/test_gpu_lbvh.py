@@ -331,3 +331,17 @@ def test_two_cloths_pairs_proximities_impacts(n):
     gi, oi = sim.impacts(1e-4), orc.impacts(1e-4)
     print("two_cloths%d impacts: gpu %d oracle %d" % (n, len(gi), len(oi)), flush=True)
     _impacts_equal(sim, orc, gi, oi)
+
+
+@pytest.mark.parametrize("sides", [(2, 3, 9), (9, 46), (47,), (2, 47, 46, 9), (33, 65, 129, 65, 129, 17)])
+def test_stages_of_small_and_large_trees(sides):
+    """Stacked sheets: up to 4,096 faces each (46: 4,050) a workgroup builds a tree, otherwise
+    (47: 4,232) the grid-wide kernels build all of them in one sort, whatever the sizes."""
+    cloths = []
+    for k, n in enumerate(sides):
+        x, f = grid_mesh(n, 0.3, origin=(1e-3 * k, 2e-3 * k, 1.2e-3 * k))
+        cloths.append(ClothSpec(MeshArrays(x, f), material_struct()))
+    sim, orc = _pair(SceneSpec("stack", default_params(dt=0.002), cloths, [], 1))
+    for case in ((False, 2e-3), (True, 1e-4)):
+        for refit in (False, True):
+            _check_pairs("stack%s" % (sides,), sim, orc, (case,), brute=False, refit=refit)

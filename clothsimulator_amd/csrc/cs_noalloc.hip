@@ -9,7 +9,11 @@
 // context's sliced ELL.  Every temporary (M^-1, r, z, d, q, partial sums, scalars) lives in
 // `scratch`, one file-scope device array of fixed size: each GPU holds its own copy for the
 // life of the process, and every call on that GPU reuses it, so calls that overlap on one GPU
-// race.  The host reads back one scalar record every NA_CHUNK iterations.
+// race.
+//
+// The iterations run in one cooperative launch (k_na_loop), a row per thread, its first blocks in
+// registers; where that launch is refused, or a wait in it runs out, as separate launches with one
+// scalar record read back every NA_CHUNK iterations.  Both give the same bits.
 #include <cfloat>
 #include <mutex>
 
@@ -40,7 +44,8 @@ constexpr size_t NA_D = NA_Z + 3 * (size_t)NA_MAX;
 constexpr size_t NA_Q = NA_D + 3 * (size_t)NA_MAX;
 constexpr size_t NA_PART = NA_Q + 3 * (size_t)NA_MAX;  // 2 floats per workgroup
 constexpr size_t NA_SCAL = NA_PART + 2 * (size_t)NA_MAXB;
-constexpr size_t NA_FLOATS = NA_SCAL + 64;
+constexpr size_t NA_SLOTS = NA_SCAL + 64;                    // 2 generations x 2 values x NA_MAXB 64-bit words
+constexpr size_t NA_FLOATS = NA_SLOTS + 8 * (size_t)NA_MAXB;
 static_assert(sizeof(NaScal) <= 64 * sizeof(float), "scalar record");
 
 // The temporaries of every call on this GPU (about 5.5 MB).  Host code never passes this name
@@ -51,6 +56,7 @@ __device__ __align__(256) float scratch[NA_FLOATS];
 struct NaPtr {
     float *Minv, *r, *z, *d, *q, *part;
     NaScal* sc;
+    uint64_t* slots;
 };
 
 NaPtr carve(float* base) {
@@ -62,6 +68,7 @@ NaPtr carve(float* base) {
     p.q = base + NA_Q;
     p.part = base + NA_PART;
     p.sc = reinterpret_cast<NaScal*>(base + NA_SCAL);
+    p.slots = reinterpret_cast<uint64_t*>(base + NA_SLOTS);
     return p;
 }
 
@@ -276,6 +283,204 @@ __global__ void k_na_clear(NaScal* sc) {
     if (threadIdx.x == 0) *sc = NaScal{};
 }
 
+// ---- the iterations in one launch ------------------------------------------
+// Separate launches take 20 us an iteration, five of them (8,100 rows of 13 blocks), all latency.  Here
+// an iteration is two meetings of the workgroups: for d.q, and for r.r and r.z, with which the new z
+// becomes visible; each thread forms its neighbours' d = z + beta d itself.
+// 8,100 rows of 13 blocks: a solve of 144 iterations 2.88 ms in separate launches, 1.44 here.
+constexpr int NA_RS = 14;                                      // blocks of a row in registers
+constexpr unsigned long long NA_WAIT_TICKS = 200000000ull;     // 2 s of the 100 MHz wall clock
+
+__device__ __forceinline__ void put1(float* p, float v) {
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// Sums v over the workgroups in the order of k_na_reduce; every thread gets them.  Each workgroup
+// stores (epoch, partial) words, every workgroup polls all of them.  Stores that a thread made with
+// put1 before the call are visible to all threads after it.  False if the wait ran out.
+template <int NS>
+__device__ bool na_meet(float (&v)[NS], int nb, unsigned ep, uint64_t* slots, int* gaveUp) {
+    __shared__ float w0[2][NA_TB / 64], w1[2][NA_TB / 64];
+    const int t = threadIdx.x, lane = t & 63, w = t >> 6;
+#pragma unroll
+    for (int s = 0; s < NS; s++) {
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) v[s] += __shfl_xor(v[s], o, 64);
+        if (lane == 0) w0[s][w] = v[s];
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's stores are out
+    __syncthreads();
+    uint64_t* gen = slots + (ep & 1) * 2 * NA_MAXB;
+    if (t < NS) {
+        float p = 0.0f;
+        for (int k = 0; k < NA_TB / 64; k++) p += w0[t][k];
+        __hip_atomic_store(gen + t * NA_MAXB + blockIdx.x, (uint64_t)ep << 32 | __float_as_uint(p), __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
+    }
+    float a[NS];
+#pragma unroll
+    for (int s = 0; s < NS; s++) a[s] = 0.0f;
+    if (t < nb) {
+        unsigned long long since = 0;
+        uint64_t word[NS];
+        for (int spin = 0;; spin++) {
+            bool all = true;
+#pragma unroll
+            for (int s = 0; s < NS; s++) {
+                word[s] = __hip_atomic_load(gen + s * NA_MAXB + t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                all = all && (unsigned)(word[s] >> 32) == ep;
+            }
+            if (all) break;
+            if ((spin & 1023) == 1023) {
+                const unsigned long long now = wall_clock64();
+                if (since == 0) since = now;
+                if (now - since > NA_WAIT_TICKS) {
+                    *gaveUp = 1;
+                    break;
+                }
+            }
+        }
+#pragma unroll
+        for (int s = 0; s < NS; s++) a[s] += __uint_as_float((unsigned)word[s]);
+    }
+#pragma unroll
+    for (int s = 0; s < NS; s++) {
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) a[s] += __shfl_xor(a[s], o, 64);
+        if (lane == 0) w1[s][w] = a[s];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int s = 0; s < NS; s++) {
+        v[s] = 0.0f;
+        for (int k = 0; k < NA_TB / 64; k++) v[s] += w1[s][k];
+    }
+    const bool ok = *gaveUp == 0;
+    if (t == 0) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");  // vectors cached before the meeting are dropped
+    __syncthreads();
+    return ok;
+}
+
+// The iterations from P's r, z = d and scalars to a stop.  nb = gridDim.x <= NA_MAXB workgroups, all
+// resident; the slots are zero at launch.  Nothing is written but P's vectors when a wait runs out.
+__global__ void __launch_bounds__(NA_TB, 2) k_na_loop(int n, const int* __restrict__ rp, const int* __restrict__ ci,
+                                                      const float* __restrict__ vals, float* __restrict__ x, NaPtr P) {
+    __shared__ int gaveUp;
+    if (P.sc->done) return;
+    if (threadIdx.x == 0) gaveUp = 0;
+    const int i = blockIdx.x * NA_TB + threadIdx.x, ic = min(i, n - 1), nb = gridDim.x;
+    const bool live = i < n;
+    const int k0 = rp[ic], k1 = live ? rp[ic + 1] : k0;
+    const float tol2bb = P.sc->tol2bb;
+    const int maxit = P.sc->maxit;
+    float rz = P.sc->rz, rr = P.sc->rr, beta = 0.0f;
+    int it = P.sc->iters;
+    const int first = it;
+    float a[NA_RS][9], m[9], xi[3], r[3], z[3], d[3], q[3];
+    unsigned short col[NA_RS];  // n <= 65,536
+#pragma unroll
+    for (int k = 0; k < NA_RS; k++) {
+        const bool in = k0 + k < k1;
+        const int kk = in ? k0 + k : rp[ic];  // (every row has its diagonal block)
+        col[k] = (unsigned short)(in ? ci[kk] : ic);
+#pragma unroll
+        for (int c = 0; c < 9; c++) {
+            const float v = vals[(size_t)kk * 9 + c];
+            a[k][c] = in ? v : 0.0f;
+        }
+    }
+#pragma unroll
+    for (int c = 0; c < 9; c++) m[c] = P.Minv[(size_t)ic * 9 + c];
+#pragma unroll
+    for (int c = 0; c < 3; c++) {
+        xi[c] = x[3 * ic + c];
+        r[c] = live ? P.r[3 * ic + c] : 0.0f;
+        z[c] = live ? P.z[3 * ic + c] : 0.0f;
+        d[c] = 0.0f;
+    }
+    unsigned ep = 0;
+    __syncthreads();
+    for (;; ) {
+        // q = A d, d = z + beta d
+        const float *dp = it & 1 ? P.d : P.q;
+        float* dn = it & 1 ? P.q : P.d;
+        auto dir = [&](int j, float (&o)[3]) {
+#pragma unroll
+            for (int c = 0; c < 3; c++) {
+                const float zj = P.z[3 * j + c];
+                o[c] = it == first ? zj : zj + beta * dp[3 * j + c];
+            }
+        };
+#pragma unroll
+        for (int c = 0; c < 3; c++) {
+            q[c] = 0.0f;
+            d[c] = it == first ? z[c] : z[c] + beta * d[c];
+        }
+        auto add = [&](const float* A, const float* v) {
+            float t[3];
+            mul3(A, v, t);
+            q[0] += t[0];
+            q[1] += t[1];
+            q[2] += t[2];
+        };
+#pragma unroll
+        for (int g = 0; g < NA_RS; g += 7) {
+            float w[7][3];
+#pragma unroll
+            for (int u = 0; u < 7; u++) dir(col[g + u], w[u]);
+#pragma unroll
+            for (int u = 0; u < 7; u++) add(a[g + u], w[u]);
+        }
+        for (int k = k0 + NA_RS; k < k1; k++) {
+            float w[3];
+            dir(ci[k], w);
+            add(vals + (size_t)k * 9, w);
+        }
+        float v1[1] = {0.0f};
+        if (live)
+#pragma unroll
+            for (int c = 0; c < 3; c++) {
+                put1(dn + 3 * i + c, d[c]);
+                v1[0] += d[c] * q[c];
+            }
+        if (!na_meet<1>(v1, nb, ++ep, P.slots, &gaveUp)) return;
+        const float alpha = rz / v1[0];
+        float v2[2] = {0.0f, 0.0f};
+#pragma unroll
+        for (int c = 0; c < 3; c++) {
+            xi[c] += alpha * d[c];
+            r[c] = live ? r[c] - alpha * q[c] : 0.0f;
+        }
+        mul3(m, r, z);
+        if (live)
+#pragma unroll
+            for (int c = 0; c < 3; c++) {
+                put1(P.z + 3 * i + c, z[c]);
+                v2[0] += r[c] * r[c];
+                v2[1] += r[c] * z[c];
+            }
+        if (!na_meet<2>(v2, nb, ++ep, P.slots, &gaveUp)) return;
+        rr = v2[0];
+        it++;
+        if (rr <= tol2bb || it >= maxit || !(rr <= FLT_MAX)) break;  // NaN: breakdown
+        beta = v2[1] / rz;
+        rz = v2[1];
+    }
+    if (live)
+#pragma unroll
+        for (int c = 0; c < 3; c++) x[3 * i + c] = xi[c];
+    if (i == 0) {
+        P.sc->rr = rr;
+        P.sc->rz = rz;
+        P.sc->iters = it;
+        P.sc->done = 1;
+    }
+}
+
+__global__ void k_na_clear_slots(uint64_t* slots) {
+    slots[blockIdx.x * NA_TB + threadIdx.x] = 0;
+}
+
 // The scratch address on each device, looked up once per device with that device current.
 std::mutex gNaMutex;
 float* gNaBase[64] = {};
@@ -293,38 +498,63 @@ float* scratch_base() {
     return gNaBase[dev];
 }
 
+// The iterations in one launch.  False: refused (another process holds the device's cooperative
+// queue, or the device has too few CUs), nothing was done.
+bool loop_at_once(hipStream_t s, int nb, int n, const int* rp, const int* ci, const float* vals, float* x, NaPtr P) {
+    hipLaunchKernelGGL(k_na_clear_slots, dim3(4 * NA_MAXB / NA_TB), dim3(NA_TB), 0, s, P.slots);
+    CS_LAUNCH_CHECK();
+    void* args[] = {(void*)&n, (void*)&rp, (void*)&ci, (void*)&vals, (void*)&x, (void*)&P};
+    if (hipLaunchCooperativeKernel((const void*)k_na_loop, dim3(nb), dim3(NA_TB), args, 0, s) == hipSuccess) return true;
+    (void)hipGetLastError();
+    return false;
+}
+
 int solve_noalloc(hipStream_t s, int n, const int* rp, const int* ci, const float* vals, const float* b, float* x,
                   float tol, int maxit, int* iters, float* relres) {
     NaPtr P = carve(scratch_base());
     const int nb = cdiv(n, NA_TB);
-    // the scalar record starts cleared: `bad` is only ever raised by the set-up kernel
-    hipLaunchKernelGGL(k_na_clear, dim3(1), dim3(64), 0, s, P.sc);
-    CS_LAUNCH_CHECK();
-    hipLaunchKernelGGL(k_na_init, dim3(nb), dim3(NA_TB), 0, s, n, rp, ci, vals, b, x, P);
-    CS_LAUNCH_CHECK();
-    hipLaunchKernelGGL(k_na_reduce, dim3(1), dim3(NA_TB), 0, s, nb, 0, tol * tol, maxit, P);
-    CS_LAUNCH_CHECK();
     NaScal h{};
+    auto start = [&]() {
+        // the scalar record starts cleared: `bad` is only ever raised by the set-up kernel
+        hipLaunchKernelGGL(k_na_clear, dim3(1), dim3(64), 0, s, P.sc);
+        CS_LAUNCH_CHECK();
+        hipLaunchKernelGGL(k_na_init, dim3(nb), dim3(NA_TB), 0, s, n, rp, ci, vals, b, x, P);
+        CS_LAUNCH_CHECK();
+        hipLaunchKernelGGL(k_na_reduce, dim3(1), dim3(NA_TB), 0, s, nb, 0, tol * tol, maxit, P);
+        CS_LAUNCH_CHECK();
+    };
     auto read = [&]() {
         CS_HIP(hipMemcpyAsync(&h, P.sc, sizeof(NaScal), hipMemcpyDeviceToHost, s));
         CS_HIP(hipStreamSynchronize(s));
     };
+    start();
+    bool once = true;
     // The loop stops on its recursive residual; as in cs_solve, only the true residual (FP64 row
     // sums) accepts the result, otherwise the loop goes on from it, at most NA_RESTARTS times.
     for (int restart = 0;; restart++) {
-        for (int done = 0; done <= maxit; done += NA_CHUNK) {
+        if (once) {
+            once = loop_at_once(s, nb, n, rp, ci, vals, x, P);
             read();
-            if (h.done) break;
-            for (int k = 0; k < NA_CHUNK; k++) {
-                hipLaunchKernelGGL(k_na_spmv, dim3(nb), dim3(NA_TB), 0, s, n, rp, ci, vals, P);
-                hipLaunchKernelGGL(k_na_reduce, dim3(1), dim3(NA_TB), 0, s, nb, 1, 0.0f, 0, P);
-                hipLaunchKernelGGL(k_na_update, dim3(nb), dim3(NA_TB), 0, s, n, x, P);
-                hipLaunchKernelGGL(k_na_reduce, dim3(1), dim3(NA_TB), 0, s, nb, 2, 0.0f, 0, P);
-                hipLaunchKernelGGL(k_na_dir, dim3(nb), dim3(NA_TB), 0, s, n, P);
+            if (once && !h.done) {  // a wait ran out: from the start
+                once = false;
+                restart = 0;
+                start();
             }
-            CS_LAUNCH_CHECK();
         }
-        read();
+        if (!once)
+            for (int done = 0; done <= maxit; done += NA_CHUNK) {
+                read();
+                if (h.done) break;
+                for (int k = 0; k < NA_CHUNK; k++) {
+                    hipLaunchKernelGGL(k_na_spmv, dim3(nb), dim3(NA_TB), 0, s, n, rp, ci, vals, P);
+                    hipLaunchKernelGGL(k_na_reduce, dim3(1), dim3(NA_TB), 0, s, nb, 1, 0.0f, 0, P);
+                    hipLaunchKernelGGL(k_na_update, dim3(nb), dim3(NA_TB), 0, s, n, x, P);
+                    hipLaunchKernelGGL(k_na_reduce, dim3(1), dim3(NA_TB), 0, s, nb, 2, 0.0f, 0, P);
+                    hipLaunchKernelGGL(k_na_dir, dim3(nb), dim3(NA_TB), 0, s, n, P);
+                }
+                CS_LAUNCH_CHECK();
+            }
+        if (!once) read();
         if (h.bad) return CS_E_ARG;
         if (!h.done) throw StatusError(CS_E_HIP, "no-allocation PCG: the device never reported its stop");
         hipLaunchKernelGGL(k_na_true, dim3(nb), dim3(NA_TB), 0, s, n, rp, ci, vals, b, x, P);

@@ -103,3 +103,32 @@ def test_noalloc_rejects_oversize_and_malformed_systems():
     # the same arrays with valid columns solve (identity system: one iteration)
     status, x, iters, _ = _noalloc(rp, np.array([0, 1], np.int32), vals, b)
     assert status == CS_OK and iters == 1 and np.allclose(x, 1.0)
+
+
+@pytest.mark.parametrize("n,reach", [(1, 0), (2, 1), (255, 3), (256, 6), (257, 7), (1000, 20), (65536, 1)])
+def test_noalloc_sizes_and_row_lengths(n, reach):
+    """One workgroup to all 256 of them; rows of up to 2 reach + 1 blocks, 14 of which are in
+    registers.  The stop is on the true residual (FP64 row sums), so in FP64 it holds up to the
+    rounding of the squared norms: 1e-5 (1 + 1e-4)."""
+    import scipy.sparse as sp
+    rng = np.random.default_rng(n + reach)
+    rp, ci, vals = [0], [], []
+    off = rng.uniform(-0.5, 0.5, (n, reach + 1))  # symmetric couplings i, i + k
+    for i in range(n):
+        for j in range(max(0, i - reach), min(n, i + reach + 1)):
+            ci.append(j)
+            vals.append(np.eye(3) * (2.0 + reach) if i == j else np.eye(3) * off[min(i, j), abs(i - j)])
+        rp.append(len(ci))
+    rp, ci = np.array(rp, np.int32), np.array(ci, np.int32)
+    vals = np.array(vals, np.float32)
+    b = rng.standard_normal(3 * n).astype(np.float32)
+    status, x, iters, rel = _noalloc(rp, ci, vals, b)
+    A = sp.bsr_matrix((vals.astype(np.float64), ci, rp), shape=(3 * n, 3 * n))
+    res = np.linalg.norm(b - A @ x.astype(np.float64)) / np.linalg.norm(b)
+    print("%d rows, reach %d: status %d, %d iterations, residual %.3g, in FP64 %.3g" % (n, reach, status, iters, rel, res))
+    assert status == CS_OK
+    assert res <= 1e-5 * (1 + 1e-4) and abs(res - rel) <= 1e-4 * rel + 1e-9
+    # the iteration budget is kept, and spending it is reported
+    if iters > 2:
+        status, x, iters, rel = _noalloc(rp, ci, vals, b, maxit=2)
+        assert status != CS_OK and iters == 2 and np.isfinite(x).all()

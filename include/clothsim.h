@@ -59,18 +59,20 @@ enum { CS_MESH_CLOTH = 0, CS_MESH_OBSTACLE = 1 };
 enum {
     CS_FLAG_NO_PROXIMITY = 1, /* skip repulsion/friction proximities (testing only; the reference always runs them) */
     CS_FLAG_NO_COLLISION = 2, /* cs_step skips the collision step (testing only) */
-    CS_FLAG_TIME_KERNELS = 4, /* sample HIP-event durations of the hot kernels (see cs_kernel_time) */
+    CS_FLAG_TIME_KERNELS = 4, /* sample HIP-event durations of the hot kernels (see cs_kernel_time); solves keep
+                                 a launch per kernel instead of one for the whole solve */
     CS_FLAG_INSTANCES = 8,    /* independent instances: cloth i collides only with itself and with obstacle i
                                  (the reference traverses every cloth pair, src/Simulator.cu:179-196, which finds
                                  nothing between instances placed apart), and with block-Jacobi PCG or
                                  CS_PRECOND_AMG all cloths' solves advance together in batched launches, each
                                  cloth with its own multigrid hierarchy, one launch per level for all of them
                                  (no counterpart) */
-    CS_FLAG_FIXED_TUNING = 16, /* batched solves keep their default launch shape instead of autotuning it
+    CS_FLAG_FIXED_TUNING = 16, /* separately launched batched solves keep their default launch shape instead of autotuning it
                                  (bit-reproducible runs; no counterpart) */
     CS_FLAG_GRAPH_CYCLES = 32, /* multigrid cycles replayed from HIP graphs captured once per solve instead of
-                                 launched kernel by kernel (the same kernels in the same order; no counterpart) */
-    CS_FLAG_PERSISTENT_BATCH = 64 /* the batched block-Jacobi solve (CS_FLAG_INSTANCES) runs the iterations between
+                                 launched kernel by kernel (the same kernels in the same order; no counterpart); also
+                                 keeps solves that would fit one launch out of it */
+    CS_FLAG_PERSISTENT_BATCH = 64 /* a batched block-Jacobi solve (CS_FLAG_INSTANCES) too large for one launch runs the iterations between
                                  two host polls as one cooperative launch, a grid barrier between the two phases
                                  of an iteration, instead of two launches per iteration (the same results bit
                                  for bit; no counterpart) */

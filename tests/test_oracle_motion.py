@@ -277,7 +277,7 @@ def strip_comments(text):
     return re.sub(r"^\s*//[^\n]*$", "", text, flags=re.M)
 
 
-@pytest.mark.skipif(not os.path.isdir(REF), reason="reference tree not present")
+@pytest.mark.skipif(not os.path.isdir(os.path.join(REF, "conf")), reason="reference tree not present")
 def test_reference_scene_motions():
     """conf/funnel.json moves the ball by a two-key smoothstep; conf/sphere.json's eight keys and
     conf/dress-blue.json's .mot bodies evaluate bit-exactly as the oracle evaluates them."""

@@ -131,7 +131,7 @@ def test_missing_mesh_file(tmp_path):
         cs.scene_info(path, str(tmp_path))
 
 
-@pytest.mark.skipif(not os.path.isdir(REF), reason="reference tree not present")
+@pytest.mark.skipif(not os.path.isdir(os.path.join(REF, "conf")), reason="reference tree not present")
 def test_reference_configurations_parse():
     """Every configuration of the reference loads (with its motions, .mot files and obstacle
     sequences), except where a file it names is not in the reference tree: conf/karate.json's

@@ -11,7 +11,7 @@ import os
 import numpy as np
 
 from ._cabi import (CS_E_COLLISION_FAILED, CS_E_NOT_CONVERGED, CS_MESH_CLOTH, CS_PRECOND_AMG_LEARNED, CS_PRECOND_LEARNED, CS_MESH_OBSTACLE, CS_OK, IMPACT_DTYPE, LIB_PATH, PROX_DTYPE,
-                    STATUS_NAMES, ImpactRec, MaterialIn, MeshArrays, MeshIn, Params, ProximityRec, SceneInfo,
+                    STATUS_NAMES, ImpactRec, LaunchFault, MaterialIn, MeshArrays, MeshIn, Params, ProximityRec, SceneInfo,
                     Remeshing, Stats, Transform, axis_angle, default_params, fptr, iptr, material_struct,
                     remeshing_struct, transform_struct)
 
@@ -25,8 +25,8 @@ EXPORTED = ["cs_version", "cs_default_params", "cs_create", "cs_destroy", "cs_la
             "cs_lbvh_pairs", "cs_find_proximities", "cs_assemble", "cs_solve", "cs_find_impacts",
             "cs_independent_impacts", "cs_kernel_time", "cs_load_scene", "cs_scene_error", "cs_precondition",
             "cs_lpc_weight_count", "cs_set_learned_weights", "cs_get_learned_weights", "cs_lpc_factor",
-            "cs_lpc_train_step", "cs_lpc_smoother_omega", "cs_batch_tuning", "cs_add_motion", "cs_motion_eval",
-            "cs_set_obstacle_motion", "cs_add_moving_handles", "cs_set_step_count", "cs_get_step_count",
+            "cs_lpc_train_step", "cs_lpc_smoother_omega", "cs_batch_tuning", "cs_solve_launches",
+            "cs_set_launch_fault", "cs_add_motion", "cs_motion_eval", "cs_set_obstacle_motion", "cs_add_moving_handles", "cs_set_step_count", "cs_get_step_count",
             "cs_scene_motion", "cs_get_topology", "cs_write_config", "cs_impact_response",
             "cs_solve_bsr_noalloc", "cs_lpc_train_step_smooth", "cs_default_remeshing", "cs_remesh_mesh",
             "cs_remesh_result_counts", "cs_remesh_result_get", "cs_remesh_result_free", "cs_set_remeshing",
@@ -94,6 +94,8 @@ def load_library(path=LIB_PATH):
     L.cs_lpc_train_step.argtypes = [vp, C.c_int, C.c_float, C.c_float, F, F]
     L.cs_lpc_train_step_smooth.argtypes = [vp, C.c_int, C.c_float, C.c_float, C.c_float, C.c_uint, F, F]
     L.cs_lpc_smoother_omega.argtypes = [vp, C.c_int, F]
+    L.cs_solve_launches.argtypes = [vp, C.POINTER(C.c_int)]
+    L.cs_set_launch_fault.argtypes = [vp, C.POINTER(LaunchFault)]
     L.cs_batch_tuning.argtypes = [vp, C.POINTER(C.c_int), C.POINTER(C.c_int), C.POINTER(C.c_int)]
     TP = C.POINTER(Transform)
     L.cs_add_motion.argtypes = [vp, F, TP, C.c_int, C.POINTER(C.c_int)]
@@ -549,6 +551,17 @@ class Simulator:
         r, c, t = C.c_int(), C.c_int(), C.c_int()
         self._check(self.L.cs_batch_tuning(self.h, C.byref(r), C.byref(c), C.byref(t)), "cs_batch_tuning")
         return r.value, c.value, t.value
+
+    def solve_launches(self):
+        """Cooperative launches that held the last solve whole (0: separate launches)."""
+        n = C.c_int()
+        self._check(self.L.cs_solve_launches(self.h, C.byref(n)), "cs_solve_launches")
+        return n.value
+
+    def set_launch_fault(self, refuse=0, lose_wg=0, lose_at=0, wait_s=0.0):
+        """How attempts at a solve in one launch go wrong (testing only; no arguments: they do not)."""
+        f = LaunchFault(refuse, lose_wg, lose_at, wait_s)
+        self._check(self.L.cs_set_launch_fault(self.h, C.byref(f)), "cs_set_launch_fault")
 
     def kernel_time(self, kernel_id, reset=False):
         """(summed ms, sampled launches) of a hot kernel; needs CS_FLAG_TIME_KERNELS in params.flags."""

@@ -124,6 +124,15 @@ class ProximityRec(C.Structure):
     ]
 
 
+class LaunchFault(C.Structure):
+    _fields_ = [
+        ("refuse", C.c_int),
+        ("lose_wg", C.c_int),
+        ("lose_at", C.c_int),
+        ("wait_s", C.c_float),
+    ]
+
+
 class ImpactRec(C.Structure):
     _fields_ = [
         ("type", C.c_int),

@@ -978,6 +978,18 @@ cs_status cs_batch_tuning(const cs_ctx* C, int* rows_per_block, int* chunk, int*
     return CS_OK;
 }
 
+cs_status cs_solve_launches(const cs_ctx* C, int* launches) {
+    if (!C || !launches) return CS_E_ARG;
+    *launches = C->ppLaunches;
+    return CS_OK;
+}
+
+cs_status cs_set_launch_fault(cs_ctx* C, const cs_launch_fault* fault) {
+    if (!C) return CS_E_ARG;
+    C->ppFault = fault ? *fault : cs_launch_fault{};
+    return CS_OK;
+}
+
 cs_status cs_lpc_smoother_omega(cs_ctx* C, int cloth_id, float* omega) {
     if (!C || !omega) return CS_E_ARG;
     if (cloth_id < 0 || cloth_id >= C->nCloths) return CS_E_ARG;

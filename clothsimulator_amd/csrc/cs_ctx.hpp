@@ -178,7 +178,8 @@ struct SepRec {
 
 struct PcgScalars {
     float rz, dq, alpha, beta, rr, bb, tol2bb, pad;
-    int iters, done, maxit, pad2;
+    int iters, done, maxit;
+    int lost;  // a workgroup of a whole solve in one launch gave up waiting: x is incomplete
 };
 
 // Sampled HIP-event timing of hot kernels (enabled by CS_FLAG_TIME_KERNELS).
@@ -251,6 +252,8 @@ struct cs_ctx {
     // whole solves in one launch (cs_ppcg.hip): system table, block -> (system, workgroup) map, slots
     cs::DBuf ppTab, ppMap, ppSlots;
     bool ppOff = false;  // refused a launch: solve with separate launches
+    int ppLaunches = 0;  // launches that held the last solve, 0: separate ones
+    cs_launch_fault ppFault{};  // (testing)
     // batched solve of independent cloths: per-cloth table, block -> cloth map, partials, scalars
     cs::DBuf bTab, bMap, bPart, bScal, bList;
     struct BatchTune {

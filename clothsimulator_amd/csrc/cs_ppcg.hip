@@ -48,7 +48,7 @@ namespace {
 
 enum { PRE_JACOBI = 0, PRE_LEARNED = 1, PRE_AMG = 2 };
 constexpr int RESTARTS = 4;                      // continuations from the true residual, as pcg_solve
-constexpr unsigned long long WAIT_TICKS = 200000000ull;  // 2 s of the 100 MHz wall clock
+constexpr unsigned long long WAIT_TICKS = 200000000ull;  // 2 s of the 100 MHz wall clock; a wait's bound
 
 // One level of a cloth's multigrid hierarchy (cs_amg.hip); agg, mptr, midx lead to the next level.
 struct PLev {
@@ -78,6 +78,7 @@ struct PSys {
     float* eBottom;
     const int *apSliceOff, *apSliceW, *apCols;
     const float* apVals;
+    int loseWg, loseAt;  // (testing) a wait of workgroup loseWg counts as run out at this meeting, 0: none
     PLev L[MAXL];
 };
 
@@ -169,10 +170,16 @@ typedef float f3n __attribute__((ext_vector_type(3)));
 
 constexpr int BLK = 256;     // rows of one partial sum
 
+// A workgroup's waits, in LDS (registers are short)
+struct Wait {
+    unsigned long long ticks;  // bound of one
+    unsigned ranOut;           // the meeting at which one ran out (they count from 1)
+};
+
 struct Group {
     G1<uint64_t>* slots;
-    float* lds;   // 2 * (T / 64 + 4) floats
-    int* gaveUp;  // LDS flag: a wait of this workgroup ran out
+    float* lds;  // 2 * (T / 64 + 4) floats
+    Wait* wait;
     int G, wg;
     unsigned epoch;
 };
@@ -228,6 +235,7 @@ __device__ __forceinline__ bool meet(Group& g, float (&v)[NS]) {
         for (int s = 0; s < NS; s++) a[s] = 0.0f;
         for (int t = 64 * c + lane; t < n; t += BLK) {
             uint64_t w[NS];
+            bool late = false;
             for (int spin = 0;; spin++) {
                 bool all = true;
 #pragma unroll
@@ -236,13 +244,14 @@ __device__ __forceinline__ bool meet(Group& g, float (&v)[NS]) {
                     all = all && (unsigned)(w[s] >> 32) == ep;
                 }
                 if (all) break;
+                if (late) {
+                    g.wait->ranOut = ep;
+                    break;
+                }
                 if ((spin & 1023) == 1023) {
                     const unsigned long long now = wall_clock64();
                     if (since == 0) since = now;
-                    if (now - since > WAIT_TICKS) {
-                        *g.gaveUp = 1;
-                        break;
-                    }
+                    late = now - since > g.wait->ticks;  // the words are read once more after the deadline
                 }
             }
 #pragma unroll
@@ -260,7 +269,7 @@ __device__ __forceinline__ bool meet(Group& g, float (&v)[NS]) {
     __syncthreads();
 #pragma unroll
     for (int s = 0; s < NS; s++) v[s] = (sums[4 * s] + sums[4 * s + 1]) + (sums[4 * s + 2] + sums[4 * s + 3]);
-    const bool ok = *g.gaveUp == 0;
+    const bool ok = g.wait->ranOut != ep;
     // vectors cached from before the meeting are dropped (one wave: the caches are the CU's and
     // the XCD's), before any thread goes on to gather
     if (PUBLISH && tid == 0) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
@@ -389,10 +398,11 @@ __device__ __forceinline__ void fromLds(const float* p, Pair& w) {
 // vectors are exchanged through LDS.  PRE: the preconditioner, as in the separate launches.
 template <int T, int RS, int GR, bool LOCAL, int PRE>
 __global__ void __launch_bounds__(T, 2)  // 256 registers: the runtime refuses cooperative kernels of more
-    k_ppcg(const PSys* __restrict__ tab, const int2* __restrict__ map, float tol2, int maxit) {
+    k_ppcg(const PSys* __restrict__ tab, const int2* __restrict__ map, float tol2, int maxit,
+           unsigned long long ticks) {
     constexpr int NW = T / 64, CN = 3, CAP = LOCAL ? 2048 : 5120;
     __shared__ float red[2 * (NW + 4)];
-    __shared__ int gaveUp;
+    __shared__ Wait wait;
     __shared__ float prod[6 * CAP];  // products of contact blocks
     __shared__ float4 zl[LOCAL ? T : 1], dl[LOCAL ? T : 1];
     constexpr bool NET = PRE == PRE_LEARNED;
@@ -407,11 +417,19 @@ __global__ void __launch_bounds__(T, 2)  // 256 registers: the runtime refuses c
     Group g;
     g.slots = S.slots;
     g.lds = red;
-    g.gaveUp = &gaveUp;
+    g.wait = &wait;
     g.G = S.G;
     g.wg = wg;
     g.epoch = 0;
-    if (tid == 0) gaveUp = 0;
+    if (tid == 0) {
+        wait.ticks = ticks;
+        wait.ranOut = P.loseWg == wg ? P.loseAt : 0;
+    }
+    // A workgroup whose wait ran out leaves the solve without its rows of x.  The others learn of it at
+    // their next meeting, but after the last one there is none: the host reads it from the record.
+    auto lost = [&]() {
+        if (tid == 0) S.out->lost = 1;
+    };
 
     const V3f zero = mk(0.0f, 0.0f, 0.0f);
     const int i = wg * T + tid, ic = min(i, nn - 1);
@@ -738,7 +756,7 @@ __global__ void __launch_bounds__(T, 2)  // 256 registers: the runtime refuses c
 
     // x = 0, r = b
     ldblk(S.Minv, row(), m);
-    if (!precondition(false)) return;
+    if (!precondition(false)) return lost();
     const float bb = rr, tol2bb = tol2 * bb;
     stop2bb = tol2bb;
     stop = bb <= tol2bb || maxit <= 0;
@@ -774,7 +792,7 @@ __global__ void __launch_bounds__(T, 2)  // 256 registers: the runtime refuses c
             }
             v1[0] = live ? dot(d, q) : 0.0f;
             if (PRE == PRE_JACOBI || PRE == PRE_AMG) ldblk(S.Minv, row(), m);  // ahead of the meeting
-            if (!meet<T, 1, false, LOCAL>(g, v1)) return;
+            if (!meet<T, 1, false, LOCAL>(g, v1)) return lost();
             const float alpha = rz / v1[0];
             if (live) {
                 x = x + alpha * d;
@@ -782,12 +800,12 @@ __global__ void __launch_bounds__(T, 2)  // 256 registers: the runtime refuses c
             }
             it++;
             rzOld = rz;
-            if (!precondition(true)) return;
+            if (!precondition(true)) return lost();
         }
         // the true residual b - A x with every row sum in FP64, the matrix from memory (once per stop)
         putZ(x);
         v1[0] = 0.0f;
-        if (!meet<T, 1, true, LOCAL>(g, v1)) return;
+        if (!meet<T, 1, true, LOCAL>(g, v1)) return lost();
         if (live) {
             double y0 = 0.0, y1 = 0.0, y2 = 0.0;
             auto put = [&](const float (&o)[9], V3f xj) {
@@ -802,14 +820,14 @@ __global__ void __launch_bounds__(T, 2)  // 256 registers: the runtime refuses c
                    (float)((double)b.z + (double)bc.z - y2));
         }
         v1[0] = dot(r, r);
-        if (!meet<T, 1, true, LOCAL>(g, v1)) return;
+        if (!meet<T, 1, true, LOCAL>(g, v1)) return lost();
         rr = v1[0];
         if (rr <= tol2bb || it >= maxit || !(rr <= FLT_MAX) || restarts == RESTARTS) break;
         // continue from it, the direction restarted from its preconditioned residual
         stop2bb = continuation_stop(tol2bb, restarts);
         stop = false;
         ldblk(S.Minv, row(), m);
-        if (!precondition(false)) return;
+        if (!precondition(false)) return lost();
     }
     if (live) {
         G1<float>* o = &at(S.x, 12u * row());
@@ -1012,8 +1030,8 @@ Plan plan_for(cs_ctx* C, const std::vector<int>& cloths, int pre, bool dense) {
     return p;
 }
 
-// Results per entry of `cloths`, as pcg_solve.  False, and nothing solved, when a launch is refused or a
-// group gives up.
+// Results per entry of `cloths`, as pcg_solve.  False, the entries of x undefined, when a launch is refused
+// or any workgroup gave up.
 bool run_plan(cs_ctx* C, const Plan& p, const std::vector<int>& cloths, int pre, bool dense, int* iters, float* relres,
               int* converged) {
     const int n = (int)cloths.size(), T = p.T;
@@ -1029,7 +1047,12 @@ bool run_plan(cs_ctx* C, const Plan& p, const std::vector<int>& cloths, int pre,
     uint64_t* slots = C->ppSlots.as<uint64_t>(words);
     PcgScalars* out = C->bScal.as<PcgScalars>(n);
     std::vector<PSys> tab(n);
-    for (int k = 0; k < n; k++) tab[k] = describe(C->sys[cloths[k]], pre, dense, G[k], slots + so[k], out + k);
+    const cs_launch_fault& fault = C->ppFault;
+    for (int k = 0; k < n; k++) {
+        tab[k] = describe(C->sys[cloths[k]], pre, dense, G[k], slots + so[k], out + k);
+        tab[k].loseWg = fault.lose_wg;
+        tab[k].loseAt = fault.lose_at;
+    }
     PSys* dtab = C->ppTab.as<PSys>(n);
     int2* dmap = C->ppMap.as<int2>(map.size());
     PcgScalars* h = static_cast<PcgScalars*>(pinned_batch(C, sizeof(PcgScalars) * n));
@@ -1039,13 +1062,15 @@ bool run_plan(cs_ctx* C, const Plan& p, const std::vector<int>& cloths, int pre,
     fill_u32(reinterpret_cast<uint32_t*>(out), 0u, (long)n * (sizeof(PcgScalars) / 4), s);
     float tol2 = C->P.pcg_rel_tol * C->P.pcg_rel_tol;
     int maxit = C->P.pcg_max_iters;
+    unsigned long long ticks = fault.wait_s > 0.0f ? (unsigned long long)(fault.wait_s * 1e8f) : WAIT_TICKS;
     for (const Round& r : p.rounds) {
         const PSys* ct = dtab;
         const int2* cm = dmap + r.off;
-        void* args[] = {(void*)&ct, (void*)&cm, (void*)&tol2, (void*)&maxit};
-        const hipError_t e = hipLaunchCooperativeKernel(p.f, dim3(r.n), dim3(T), args, 0, s);
+        void* args[] = {(void*)&ct, (void*)&cm, (void*)&tol2, (void*)&maxit, (void*)&ticks};
+        const hipError_t e = fault.refuse ? hipErrorCooperativeLaunchTooLarge
+                                          : hipLaunchCooperativeKernel(p.f, dim3(r.n), dim3(T), args, 0, s);
         if (e != hipSuccess) {
-                // too large, or another process holds the device's cooperative queue
+            // too large, or another process holds the device's cooperative queue
             (void)hipGetLastError();
             CS_HIP(hipStreamSynchronize(s));
             C->ppOff = true;
@@ -1055,7 +1080,7 @@ bool run_plan(cs_ctx* C, const Plan& p, const std::vector<int>& cloths, int pre,
     CS_HIP(hipMemcpyAsync(h, out, sizeof(PcgScalars) * n, hipMemcpyDeviceToHost, s));
     CS_HIP(hipStreamSynchronize(s));
     for (int k = 0; k < n; k++)
-        if (!h[k].done) {
+        if (!h[k].done || h[k].lost) {
             C->ppOff = true;
             return false;
         }
@@ -1065,6 +1090,7 @@ bool run_plan(cs_ctx* C, const Plan& p, const std::vector<int>& cloths, int pre,
         converged[k] = h[k].rr <= h[k].tol2bb;
         C->sys[cloths[k]].solved = converged[k] != 0;
     }
+    C->ppLaunches += (int)p.rounds.size();
     return true;
 }
 
@@ -1075,6 +1101,7 @@ bool allowed(const cs_ctx* C) {
 }  // namespace
 
 bool ppcg_solve(cs_ctx* C, int c, bool amg, bool learned, int* iters, float* relres, int* converged) {
+    C->ppLaunches = 0;
     // the cycle with the learned smoother would meet 13 times an iteration: measured slower at every size
     if (!allowed(C) || (amg && learned)) return false;
     const int pre = amg ? PRE_AMG : learned ? PRE_LEARNED : PRE_JACOBI;
@@ -1084,6 +1111,7 @@ bool ppcg_solve(cs_ctx* C, int c, bool amg, bool learned, int* iters, float* rel
 }
 
 bool ppcg_solve_batch(cs_ctx* C, bool amg, int* iters, float* relres, int* converged) {
+    C->ppLaunches = 0;
     if (!allowed(C)) return false;
     std::vector<int> part[2];  // block Jacobi, multigrid
     const std::vector<int>* usable = amg ? &bamg_build(C) : nullptr;
@@ -1100,8 +1128,10 @@ bool ppcg_solve_batch(cs_ctx* C, bool amg, int* iters, float* relres, int* conve
         const int n = (int)part[k].size();
         std::vector<int> it(n), cv(n);
         std::vector<float> rel(n);
-        if (!run_plan(C, plan[k], part[k], k ? PRE_AMG : PRE_JACOBI, false, it.data(), rel.data(), cv.data()))
+        if (!run_plan(C, plan[k], part[k], k ? PRE_AMG : PRE_JACOBI, false, it.data(), rel.data(), cv.data())) {
+            C->ppLaunches = 0;
             return false;
+        }
         for (int j = 0; j < n; j++) {
             iters[part[k][j]] = it[j];
             relres[part[k][j]] = rel[j];

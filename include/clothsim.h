@@ -327,6 +327,20 @@ cs_status cs_lpc_smoother_omega(cs_ctx* ctx, int cloth_id, float* omega);
  * autotuner has timed so far (it settles after 8).  No counterpart in the reference. */
 cs_status cs_batch_tuning(const cs_ctx* ctx, int* rows_per_block, int* chunk, int* trials);
 
+/* The cooperative launches that held the context's last solve whole: 1, or more for a batch; 0 when it
+ * ran in separate launches.  No counterpart in the reference. */
+cs_status cs_solve_launches(const cs_ctx* ctx, int* launches);
+/* How the attempts at a solve in one launch go wrong (testing only; all zero: they do not).  The results
+ * are those of separate launches either way. */
+typedef struct cs_launch_fault {
+    int refuse;  /* 1: every such launch counts as refused */
+    int lose_wg, lose_at; /* a wait of workgroup lose_wg counts as run out at its lose_at-th meeting (from 1) with
+                             the solve's other workgroups; 0: none */
+    float wait_s; /* > 0: a wait's bound (s); 2 otherwise */
+} cs_launch_fault;
+/* Sets (fault != NULL) or clears the context's fault, for its next solves. */
+cs_status cs_set_launch_fault(cs_ctx* ctx, const cs_launch_fault* fault);
+
 /* Simulator::findImpacts (src/Simulator.cu:383-392), deduplicated and sorted by (t, type, nodes). */
 cs_status cs_find_impacts(cs_ctx* ctx, float thickness, cs_impact_rec* out, int cap, int* n_out);
 /* Simulator::independentImpacts GPU (src/Simulator.cu:422-461) on caller-provided impacts

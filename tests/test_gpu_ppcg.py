@@ -174,3 +174,69 @@ def test_two_runs_give_the_same_bits():
     a, _, _ = _solve(spec, 0, x, v)
     b, _, _ = _solve(spec, 0, x, v)
     assert np.array_equal(a, b)
+
+
+def _fault_case(case):
+    """(spec, two states) of a system in the one-launch range with several workgroups."""
+    if case == "batch":
+        spec = scenes.instances(count=3, seed=3, side_lo=23, side_hi=40)
+        spec.params.flags |= CS_FLAG_FIXED_TUNING
+        return spec
+    spec = scenes.crumple(33, height=0.01, sigma=0.05 / 33)
+    spec.params.precond = {"jacobi": 0, "learned": CS_PRECOND_LEARNED, "amg": CS_PRECOND_AMG}[case]
+    return spec
+
+
+def _solve_after_another(case, flags=0, **fault):
+    """A solve right after one of another system on the same context (what it leaves in the buffers is
+    no solution here): (solution, iterations, launches)."""
+    spec = _fault_case(case)
+    spec.params.flags |= flags
+    sim = Simulator(spec)
+    for seed in (1, 2):
+        rng = np.random.default_rng(seed)
+        for k in range(sim.n_cloths):
+            x = sim.state(CS_MESH_CLOTH, k)[0]
+            sim.set_state(CS_MESH_CLOTH, k, x, x, np.float32(rng.normal(0, 0.2, x.shape)))
+        if seed == 2:
+            assert sim.solve_launches() == (0 if flags else 1)
+            sim.set_launch_fault(**fault)
+        if case == "batch":
+            s, st = sim.physics_step()
+            assert s == 0
+            dv = np.concatenate([sim.state(CS_MESH_CLOTH, k)[2].ravel() for k in range(sim.n_cloths)])
+        else:
+            sim.assemble(0)
+            dv, st = sim.solve(0)
+        assert st.pcg_converged
+    return dv, st.pcg_iters, sim.solve_launches()
+
+
+@pytest.mark.parametrize("case", ["jacobi", "learned", "amg", "batch"])
+def test_a_refused_launch_falls_back(case):
+    dv, it, launches = _solve_after_another(case, refuse=1)
+    ref, rit, _ = _solve_after_another(case, CS_FLAG_TIME_KERNELS)
+    assert launches == 0 and it == rit and np.array_equal(dv, ref)
+
+
+@pytest.mark.parametrize("case", ["jacobi", "learned", "amg", "batch"])
+@pytest.mark.parametrize("at", [1, 2, 7, 30])
+def test_a_workgroup_that_gives_up_falls_back(case, at):
+    """Its peers' next wait runs out (bounded to 5 ms here); the solve is repeated in separate launches."""
+    dv, it, launches = _solve_after_another(case, lose_wg=1, lose_at=at, wait_s=5e-3)
+    ref, rit, _ = _solve_after_another(case, CS_FLAG_TIME_KERNELS)
+    assert launches == 0 and it == rit and np.array_equal(dv, ref)
+
+
+def test_a_workgroup_that_gives_up_at_the_last_meeting_is_noticed():
+    """At the last meeting no peer waits for the lost workgroup again, and the record is complete: only
+    the lost workgroup's own word tells.  A block-Jacobi solve of i iterations meets 2 i + 3 times, and
+    three times more per continuation from the true residual."""
+    ref, it, _ = _solve_after_another("jacobi", CS_FLAG_TIME_KERNELS)
+    ran = []
+    for at in [2 * it + 3 + 3 * k for k in range(5)] + [2 * it + 4 + 3 * k for k in range(5)]:
+        dv, i, launches = _solve_after_another("jacobi", lose_wg=1, lose_at=at, wait_s=5e-3)
+        assert i == it and np.array_equal(dv, ref), at
+        ran.append((at, launches))
+    last = max(at for at, launches in ran if launches == 0)
+    assert (last + 1, 1) in ran  # one later is never reached: `last` was the last meeting

@@ -1460,7 +1460,7 @@ static void solve_batched(cs_ctx* C, int chunk, int* iters, float* relres, int* 
     }
 }
 
-// Batched-solve autotuner: the first solves of a context try every (rows per
+// Batched-solve autotuner: the first separately launched solves of a context try every (rows per
 // block, iterations per poll) candidate twice, round robin, and score each by
 // host wall time per node-iteration (sum over cloths of iterations x rows); the
 // best is kept for the context's later solves.  The rows per block set the
@@ -1474,6 +1474,9 @@ constexpr int kTuneN = 4, kTuneRounds = 2;
 // each cloth's multigrid cycle).  Per cloth: iterations, relative residual and convergence,
 // as pcg_solve.  A multigrid iteration costs several Jacobi ones, so it polls a quarter as often.
 void pcg_solve_batched(cs_ctx* C, int* iters, float* relres, int* converged, bool amg) {
+    // every cloth's whole solve inside one or two launches where the matrices fit the chip (no candidate
+    // applies there, so none is tried or scored: the results are those of 256 rows, bit for bit)
+    if (ppcg_solve_batch(C, amg, iters, relres, converged)) return;
     auto& T = C->batchTune;
     int cand = T.choice;
     const bool tuning = !(C->P.flags & CS_FLAG_FIXED_TUNING) && T.trials < kTuneN * kTuneRounds;
@@ -1481,11 +1484,7 @@ void pcg_solve_batched(cs_ctx* C, int* iters, float* relres, int* converged, boo
     else if (tuning) cand = T.trials % kTuneN;
     const auto t0 = std::chrono::steady_clock::now();
     const int chunk = amg ? kTuneChunk[cand] / 4 : kTuneChunk[cand];
-    // every cloth's whole solve inside one or two launches where the matrices fit the chip (no
-    // candidate applies there: the results are those of 256 rows, bit for bit)
-    const bool onchip = ppcg_solve_batch(C, amg, iters, relres, converged);
-    if (onchip) {
-    } else if (kTuneRows[cand] == 128) solve_batched<128>(C, chunk, iters, relres, converged, amg);
+    if (kTuneRows[cand] == 128) solve_batched<128>(C, chunk, iters, relres, converged, amg);
     else solve_batched<256>(C, chunk, iters, relres, converged, amg);
     if (tuning) {
         const double sec = std::chrono::duration<double>(std::chrono::steady_clock::now() - t0).count();

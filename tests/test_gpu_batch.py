@@ -5,7 +5,8 @@ import numpy as np
 import pytest
 
 from clothsimulator_amd import CS_MESH_CLOTH, Simulator, scenes
-from clothsimulator_amd._cabi import CS_FLAG_FIXED_TUNING, CS_FLAG_INSTANCES, CS_FLAG_PERSISTENT_BATCH
+from clothsimulator_amd._cabi import (CS_FLAG_FIXED_TUNING, CS_FLAG_INSTANCES, CS_FLAG_PERSISTENT_BATCH,
+                                      CS_FLAG_TIME_KERNELS)
 
 pytestmark = pytest.mark.gpu
 
@@ -115,13 +116,16 @@ def test_instance_pairs_stay_inside_their_instance():
 
 
 def test_batched_solve_autotuner_settles():
-    """The batched solve times its candidate launch shapes over the first 8 solves and keeps
-    one; with CS_FLAG_FIXED_TUNING it keeps (256 rows, 16 iterations per poll)."""
+    """The batched solve times its candidate launch shapes over the first 8 separately launched solves
+    (CS_FLAG_TIME_KERNELS keeps this batch there) and keeps one; with CS_FLAG_FIXED_TUNING it keeps (256
+    rows, 16 iterations per poll)."""
     spec = scenes.instances(count=6, seed=7, side_lo=17, side_hi=33)
+    spec.params.flags |= CS_FLAG_TIME_KERNELS
     sim = Simulator(spec)
     for k in range(10):
         s, st = sim.step()
         assert s == 0, s
+    assert sim.solve_launches() == 0
     rows, chunk, trials = sim.batch_tuning()
     print("tuned: %d rows per block, %d iterations per poll after %d timed solves" % (rows, chunk, trials))
     assert trials == 8 and rows in (128, 256) and chunk in (16, 32)
@@ -131,6 +135,20 @@ def test_batched_solve_autotuner_settles():
         s, st = fixed.step()
         assert s == 0, s
     assert fixed.batch_tuning() == (256, 16, 0)
+
+
+def test_solves_in_one_launch_are_no_trials():
+    """A batch whose solves run in one launch tries no launch shape; the first launched solve does."""
+    spec = scenes.instances(count=6, seed=7, side_lo=17, side_hi=33)
+    sim = Simulator(spec)
+    for k in range(10):
+        s, st = sim.step()
+        assert s == 0 and sim.solve_launches() == 1
+    assert sim.batch_tuning() == (256, 16, 0)
+    sim.set_launch_fault(refuse=1)
+    s, st = sim.step()
+    assert s == 0 and sim.solve_launches() == 0
+    assert sim.batch_tuning()[2] == 1
 
 
 def test_batch32_up_to_side129_matches_separate_runs_and_oracle():

@@ -28,7 +28,8 @@ EXPORTED = ["cs_version", "cs_default_params", "cs_create", "cs_destroy", "cs_la
             "cs_lpc_train_step", "cs_lpc_smoother_omega", "cs_batch_tuning", "cs_solve_launches",
             "cs_set_launch_fault", "cs_add_motion", "cs_motion_eval", "cs_set_obstacle_motion", "cs_add_moving_handles", "cs_set_step_count", "cs_get_step_count",
             "cs_scene_motion", "cs_get_topology", "cs_write_config", "cs_impact_response",
-            "cs_solve_bsr_noalloc", "cs_lpc_train_step_smooth", "cs_default_remeshing", "cs_remesh_mesh",
+            "cs_solve_bsr_noalloc", "cs_solve_bsr_noalloc_test", "cs_lpc_train_step_smooth",
+            "cs_default_remeshing", "cs_remesh_mesh",
             "cs_remesh_result_counts", "cs_remesh_result_get", "cs_remesh_result_free", "cs_set_remeshing",
             "cs_remesh", "cs_remesh_sizing", "cs_remesh_times", "cs_separation_step", "cs_frame_begin",
             "cs_frame_end"]
@@ -82,6 +83,7 @@ def load_library(path=LIB_PATH):
                                          C.POINTER(C.c_int)]
     L.cs_solve_bsr_noalloc.argtypes = [vp, C.c_int, vp, vp, vp, vp, vp, C.c_float, C.c_int, C.POINTER(C.c_int),
                                        C.POINTER(C.c_float)]
+    L.cs_solve_bsr_noalloc_test.argtypes = L.cs_solve_bsr_noalloc.argtypes + [C.POINTER(LaunchFault), C.POINTER(C.c_int)]
     L.cs_impact_response.argtypes = [vp, C.POINTER(ImpactRec), C.c_int, C.c_int, C.c_float, C.POINTER(C.c_int)]
     L.cs_kernel_time.argtypes = [vp, C.c_int, C.POINTER(C.c_double), C.POINTER(C.c_int), C.c_int]
     L.cs_load_scene.argtypes = [C.c_char_p, C.c_char_p, C.POINTER(Params), C.POINTER(vp), C.POINTER(SceneInfo)]

@@ -34,6 +34,7 @@ constexpr int NA_RESTARTS = 4;                // continuations from the true res
 struct NaScal {
     float bb, rz, rr, alpha, beta, tol2bb;
     int done, iters, maxit, bad;
+    int lost;  // a workgroup of k_na_loop gave up waiting: x is incomplete
 };
 
 // float offsets into the scratch array
@@ -57,10 +58,12 @@ struct NaPtr {
     float *Minv, *r, *z, *d, *q, *part;
     NaScal* sc;
     uint64_t* slots;
+    unsigned long long ticks;  // bound of a wait of k_na_loop
+    int loseWg, loseAt;        // (testing) a wait of workgroup loseWg counts as run out at this meeting, 0: none
 };
 
 NaPtr carve(float* base) {
-    NaPtr p;
+    NaPtr p{};
     p.Minv = base + NA_MINV;
     p.r = base + NA_R;
     p.z = base + NA_Z;
@@ -289,7 +292,7 @@ __global__ void k_na_clear(NaScal* sc) {
 // becomes visible; each thread forms its neighbours' d = z + beta d itself.
 // 8,100 rows of 13 blocks: a solve of 144 iterations 2.88 ms in separate launches, 1.44 here.
 constexpr int NA_RS = 14;                                      // blocks of a row in registers
-constexpr unsigned long long NA_WAIT_TICKS = 200000000ull;     // 2 s of the 100 MHz wall clock
+constexpr unsigned long long NA_WAIT_TICKS = 200000000ull;     // 2 s of the 100 MHz wall clock; a wait's bound
 
 __device__ __forceinline__ void put1(float* p, float v) {
     __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -297,9 +300,10 @@ __device__ __forceinline__ void put1(float* p, float v) {
 
 // Sums v over the workgroups in the order of k_na_reduce; every thread gets them.  Each workgroup
 // stores (epoch, partial) words, every workgroup polls all of them.  Stores that a thread made with
-// put1 before the call are visible to all threads after it.  False if the wait ran out.
+// put1 before the call are visible to all threads after it.  False if the wait ran out; *ranOut (LDS) is the
+// meeting at which one did (they count from 1).
 template <int NS>
-__device__ bool na_meet(float (&v)[NS], int nb, unsigned ep, uint64_t* slots, int* gaveUp) {
+__device__ bool na_meet(float (&v)[NS], int nb, unsigned ep, const NaPtr& P, unsigned* ranOut) {
     __shared__ float w0[2][NA_TB / 64], w1[2][NA_TB / 64];
     const int t = threadIdx.x, lane = t & 63, w = t >> 6;
 #pragma unroll
@@ -310,7 +314,7 @@ __device__ bool na_meet(float (&v)[NS], int nb, unsigned ep, uint64_t* slots, in
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // this wave's stores are out
     __syncthreads();
-    uint64_t* gen = slots + (ep & 1) * 2 * NA_MAXB;
+    uint64_t* gen = P.slots + (ep & 1) * 2 * NA_MAXB;
     if (t < NS) {
         float p = 0.0f;
         for (int k = 0; k < NA_TB / 64; k++) p += w0[t][k];
@@ -323,6 +327,7 @@ __device__ bool na_meet(float (&v)[NS], int nb, unsigned ep, uint64_t* slots, in
     if (t < nb) {
         unsigned long long since = 0;
         uint64_t word[NS];
+        bool late = false;
         for (int spin = 0;; spin++) {
             bool all = true;
 #pragma unroll
@@ -331,13 +336,14 @@ __device__ bool na_meet(float (&v)[NS], int nb, unsigned ep, uint64_t* slots, in
                 all = all && (unsigned)(word[s] >> 32) == ep;
             }
             if (all) break;
+            if (late) {
+                *ranOut = ep;
+                break;
+            }
             if ((spin & 1023) == 1023) {
                 const unsigned long long now = wall_clock64();
                 if (since == 0) since = now;
-                if (now - since > NA_WAIT_TICKS) {
-                    *gaveUp = 1;
-                    break;
-                }
+                late = now - since > P.ticks;  // the words are read once more after the deadline
             }
         }
 #pragma unroll
@@ -355,19 +361,23 @@ __device__ bool na_meet(float (&v)[NS], int nb, unsigned ep, uint64_t* slots, in
         v[s] = 0.0f;
         for (int k = 0; k < NA_TB / 64; k++) v[s] += w1[s][k];
     }
-    const bool ok = *gaveUp == 0;
+    const bool ok = *ranOut != ep;
     if (t == 0) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");  // vectors cached before the meeting are dropped
     __syncthreads();
     return ok;
 }
 
 // The iterations from P's r, z = d and scalars to a stop.  nb = gridDim.x <= NA_MAXB workgroups, all
-// resident; the slots are zero at launch.  Nothing is written but P's vectors when a wait runs out.
+// resident; the slots are zero at launch.  A workgroup whose wait runs out leaves without its rows of x
+// and says so in P's record: after the last meeting no other would notice.
 __global__ void __launch_bounds__(NA_TB, 2) k_na_loop(int n, const int* __restrict__ rp, const int* __restrict__ ci,
                                                       const float* __restrict__ vals, float* __restrict__ x, NaPtr P) {
-    __shared__ int gaveUp;
+    __shared__ unsigned ranOut;
     if (P.sc->done) return;
-    if (threadIdx.x == 0) gaveUp = 0;
+    if (threadIdx.x == 0) ranOut = P.loseWg == (int)blockIdx.x ? P.loseAt : 0;
+    auto lost = [&]() {
+        if (threadIdx.x == 0) P.sc->lost = 1;
+    };
     const int i = blockIdx.x * NA_TB + threadIdx.x, ic = min(i, n - 1), nb = gridDim.x;
     const bool live = i < n;
     const int k0 = rp[ic], k1 = live ? rp[ic + 1] : k0;
@@ -443,7 +453,7 @@ __global__ void __launch_bounds__(NA_TB, 2) k_na_loop(int n, const int* __restri
                 put1(dn + 3 * i + c, d[c]);
                 v1[0] += d[c] * q[c];
             }
-        if (!na_meet<1>(v1, nb, ++ep, P.slots, &gaveUp)) return;
+        if (!na_meet<1>(v1, nb, ++ep, P, &ranOut)) return lost();
         const float alpha = rz / v1[0];
         float v2[2] = {0.0f, 0.0f};
 #pragma unroll
@@ -459,7 +469,7 @@ __global__ void __launch_bounds__(NA_TB, 2) k_na_loop(int n, const int* __restri
                 v2[0] += r[c] * r[c];
                 v2[1] += r[c] * z[c];
             }
-        if (!na_meet<2>(v2, nb, ++ep, P.slots, &gaveUp)) return;
+        if (!na_meet<2>(v2, nb, ++ep, P, &ranOut)) return lost();
         rr = v2[0];
         it++;
         if (rr <= tol2bb || it >= maxit || !(rr <= FLT_MAX)) break;  // NaN: breakdown
@@ -500,7 +510,9 @@ float* scratch_base() {
 
 // The iterations in one launch.  False: refused (another process holds the device's cooperative
 // queue, or the device has too few CUs), nothing was done.
-bool loop_at_once(hipStream_t s, int nb, int n, const int* rp, const int* ci, const float* vals, float* x, NaPtr P) {
+bool loop_at_once(hipStream_t s, int nb, int n, const int* rp, const int* ci, const float* vals, float* x, NaPtr P,
+                  bool refuse) {
+    if (refuse) return false;
     hipLaunchKernelGGL(k_na_clear_slots, dim3(4 * NA_MAXB / NA_TB), dim3(NA_TB), 0, s, P.slots);
     CS_LAUNCH_CHECK();
     void* args[] = {(void*)&n, (void*)&rp, (void*)&ci, (void*)&vals, (void*)&x, (void*)&P};
@@ -510,8 +522,11 @@ bool loop_at_once(hipStream_t s, int nb, int n, const int* rp, const int* ci, co
 }
 
 int solve_noalloc(hipStream_t s, int n, const int* rp, const int* ci, const float* vals, const float* b, float* x,
-                  float tol, int maxit, int* iters, float* relres) {
+                  float tol, int maxit, int* iters, float* relres, const cs_launch_fault& fault, int* launches) {
     NaPtr P = carve(scratch_base());
+    P.ticks = fault.wait_s > 0.0f ? (unsigned long long)(fault.wait_s * 1e8f) : NA_WAIT_TICKS;
+    P.loseWg = fault.lose_wg;
+    P.loseAt = fault.lose_at;
     const int nb = cdiv(n, NA_TB);
     NaScal h{};
     auto start = [&]() {
@@ -529,13 +544,14 @@ int solve_noalloc(hipStream_t s, int n, const int* rp, const int* ci, const floa
     };
     start();
     bool once = true;
+    int restart = 0;
     // The loop stops on its recursive residual; as in cs_solve, only the true residual (FP64 row
     // sums) accepts the result, otherwise the loop goes on from it, at most NA_RESTARTS times.
-    for (int restart = 0;; restart++) {
+    for (;; restart++) {
         if (once) {
-            once = loop_at_once(s, nb, n, rp, ci, vals, x, P);
+            once = loop_at_once(s, nb, n, rp, ci, vals, x, P, fault.refuse != 0);
             read();
-            if (once && !h.done) {  // a wait ran out: from the start
+            if (once && (!h.done || h.lost)) {  // a wait ran out: from the start
                 once = false;
                 restart = 0;
                 start();
@@ -565,6 +581,7 @@ int solve_noalloc(hipStream_t s, int n, const int* rp, const int* ci, const floa
     }
     if (iters) *iters = h.iters;
     if (relres) *relres = h.bb > 0.0f ? sqrtf(h.rr / h.bb) : 0.0f;
+    if (launches) *launches = once ? 1 + restart : 0;
     return h.rr <= h.tol2bb ? CS_OK : CS_E_NOT_CONVERGED;
 }
 
@@ -575,13 +592,22 @@ int solve_noalloc(hipStream_t s, int n, const int* rp, const int* ci, const floa
 extern "C" cs_status cs_solve_bsr_noalloc(void* stream, int n_nodes, const int* row_ptr, const int* col_idx,
                                           const float* vals, const float* b, float* x, float rel_tol, int max_iters,
                                           int* iters, float* rel_residual) {
+    return cs_solve_bsr_noalloc_test(stream, n_nodes, row_ptr, col_idx, vals, b, x, rel_tol, max_iters, iters,
+                                     rel_residual, nullptr, nullptr);
+}
+
+extern "C" cs_status cs_solve_bsr_noalloc_test(void* stream, int n_nodes, const int* row_ptr, const int* col_idx,
+                                               const float* vals, const float* b, float* x, float rel_tol,
+                                               int max_iters, int* iters, float* rel_residual,
+                                               const cs_launch_fault* fault, int* launches) {
     if (n_nodes > CS_NOALLOC_MAX_NODES) return CS_E_CAPACITY;
     if (n_nodes < 1 || !row_ptr || !col_idx || !vals || !b || !x || !(rel_tol > 0.0f) || !(rel_tol < 1.0f) ||
         max_iters < 0)
         return CS_E_ARG;
     try {
         return static_cast<cs_status>(cs::solve_noalloc(static_cast<hipStream_t>(stream), n_nodes, row_ptr, col_idx,
-                                                        vals, b, x, rel_tol, max_iters, iters, rel_residual));
+                                                        vals, b, x, rel_tol, max_iters, iters, rel_residual,
+                                                        fault ? *fault : cs_launch_fault{}, launches));
     } catch (const cs::StatusError& e) {
         return static_cast<cs_status>(e.status);
     } catch (const std::exception&) {

@@ -272,6 +272,14 @@ cs_status cs_assemble(cs_ctx* ctx, int cloth_id, int* row_ptr, int* col_idx, flo
                       int* nnzb_out, float* b);
 /* Solve the last assembled system of one cloth (src/Cloth.cu:766-809): dv (3n). */
 cs_status cs_solve(cs_ctx* ctx, int cloth_id, float* dv, cs_stats* stats);
+/* How the attempts at a solve in one launch go wrong (testing only; all zero: they do not).  The results
+ * are those of separate launches either way. */
+typedef struct cs_launch_fault {
+    int refuse;  /* 1: every such launch counts as refused */
+    int lose_wg, lose_at; /* a wait of workgroup lose_wg counts as run out at its lose_at-th meeting (from 1) with
+                             the solve's other workgroups; 0: none */
+    float wait_s; /* > 0: a wait's bound (s); 2 otherwise */
+} cs_launch_fault;
 /* ---- solve without allocation.  No counterpart in the reference: for callers that cannot
  * allocate device memory (code under HIP graph capture, tight serving loops, harnesses that
  * forbid hipMalloc).  The block-Jacobi PCG of cs_solve (x = 0, same iteration, stop when
@@ -289,6 +297,11 @@ cs_status cs_solve(cs_ctx* ctx, int cloth_id, float* dv, cs_stats* stats);
 cs_status cs_solve_bsr_noalloc(void* stream, int n_nodes, const int* row_ptr, const int* col_idx, const float* vals,
                                const float* b, float* x, float rel_tol, int max_iters, int* iters,
                                float* rel_residual);
+/* The same with a fault (NULL: none; testing only); launches (may be NULL): the cooperative launches that held
+ * the iterations, 0 when they ran in separate launches. */
+cs_status cs_solve_bsr_noalloc_test(void* stream, int n_nodes, const int* row_ptr, const int* col_idx,
+                                    const float* vals, const float* b, float* x, float rel_tol, int max_iters,
+                                    int* iters, float* rel_residual, const cs_launch_fault* fault, int* launches);
 /* The CS_PRECOND_AMG, CS_PRECOND_LEARNED or CS_PRECOND_AMG_LEARNED preconditioner of the last
  * assembled system (no counterpart in the reference, whose PCG uses the Jacobi diagonal): the
  * level sizes of the multigrid hierarchy (n_levels = 0 when the cloth cannot use it; always 0
@@ -330,14 +343,6 @@ cs_status cs_batch_tuning(const cs_ctx* ctx, int* rows_per_block, int* chunk, in
 /* The cooperative launches that held the context's last solve whole: 1, or more for a batch; 0 when it
  * ran in separate launches.  No counterpart in the reference. */
 cs_status cs_solve_launches(const cs_ctx* ctx, int* launches);
-/* How the attempts at a solve in one launch go wrong (testing only; all zero: they do not).  The results
- * are those of separate launches either way. */
-typedef struct cs_launch_fault {
-    int refuse;  /* 1: every such launch counts as refused */
-    int lose_wg, lose_at; /* a wait of workgroup lose_wg counts as run out at its lose_at-th meeting (from 1) with
-                             the solve's other workgroups; 0: none */
-    float wait_s; /* > 0: a wait's bound (s); 2 otherwise */
-} cs_launch_fault;
 /* Sets (fault != NULL) or clears the context's fault, for its next solves. */
 cs_status cs_set_launch_fault(cs_ctx* ctx, const cs_launch_fault* fault);
 

@@ -14,7 +14,7 @@ import numpy as np
 import pytest
 
 from clothsimulator_amd import Simulator, load_library, scenes
-from clothsimulator_amd._cabi import CS_E_ARG, CS_E_CAPACITY, CS_OK
+from clothsimulator_amd._cabi import CS_E_ARG, CS_E_CAPACITY, CS_OK, LaunchFault
 
 pytestmark = pytest.mark.gpu
 
@@ -49,15 +49,24 @@ class DeviceArray:
         self.H.hipFree(self.ptr)
 
 
-def _noalloc(rp, ci, vals, b, tol=1e-5, maxit=4000):
-    L = load_library()
+def _noalloc(rp, ci, vals, b, tol=1e-5, maxit=4000, entry="cs_solve_bsr_noalloc", more=()):
+    """(status, x, iterations, residual)"""
+    solve = getattr(load_library(), entry)
     drp, dci = DeviceArray(rp.astype(np.int32)), DeviceArray(ci.astype(np.int32))
     dvals, db = DeviceArray(vals.reshape(-1).astype(np.float32)), DeviceArray(b.astype(np.float32))
     dx = DeviceArray(np.full(len(b), np.nan, np.float32))
     it, rel = C.c_int(-1), C.c_float(-1.0)
-    st = L.cs_solve_bsr_noalloc(None, len(rp) - 1, drp.ptr, dci.ptr, dvals.ptr, db.ptr, dx.ptr, tol, maxit,
-                                C.byref(it), C.byref(rel))
+    st = solve(None, len(rp) - 1, drp.ptr, dci.ptr, dvals.ptr, db.ptr, dx.ptr, tol, maxit, C.byref(it), C.byref(rel),
+               *more)
     return st, dx.get(), it.value, rel.value
+
+
+def _noalloc_launches(rp, ci, vals, b, **fault):
+    """(status, x, iterations, residual, launches that held the iterations); fault: how the launch fails."""
+    launches = C.c_int(-1)
+    out = _noalloc(rp, ci, vals, b, entry="cs_solve_bsr_noalloc_test",
+                   more=(C.byref(LaunchFault(**fault)), C.byref(launches)))
+    return *out, launches.value
 
 
 def test_noalloc_solve_matches_cs_solve_on_two_calls():
@@ -105,12 +114,8 @@ def test_noalloc_rejects_oversize_and_malformed_systems():
     assert status == CS_OK and iters == 1 and np.allclose(x, 1.0)
 
 
-@pytest.mark.parametrize("n,reach", [(1, 0), (2, 1), (255, 3), (256, 6), (257, 7), (1000, 20), (65536, 1)])
-def test_noalloc_sizes_and_row_lengths(n, reach):
-    """One workgroup to all 256 of them; rows of up to 2 reach + 1 blocks, 14 of which are in
-    registers.  The stop is on the true residual (FP64 row sums), so in FP64 it holds up to the
-    rounding of the squared norms: 1e-5 (1 + 1e-4)."""
-    import scipy.sparse as sp
+def _band(n, reach):
+    """A symmetric, diagonally dominant system with rows of up to 2 reach + 1 blocks."""
     rng = np.random.default_rng(n + reach)
     rp, ci, vals = [0], [], []
     off = rng.uniform(-0.5, 0.5, (n, reach + 1))  # symmetric couplings i, i + k
@@ -122,7 +127,18 @@ def test_noalloc_sizes_and_row_lengths(n, reach):
     rp, ci = np.array(rp, np.int32), np.array(ci, np.int32)
     vals = np.array(vals, np.float32)
     b = rng.standard_normal(3 * n).astype(np.float32)
-    status, x, iters, rel = _noalloc(rp, ci, vals, b)
+    return rp, ci, vals, b
+
+
+@pytest.mark.parametrize("n,reach", [(1, 0), (2, 1), (255, 3), (256, 6), (257, 7), (1000, 20), (65536, 1)])
+def test_noalloc_sizes_and_row_lengths(n, reach):
+    """One workgroup to all 256 of them; rows of up to 2 reach + 1 blocks, 14 of which are in
+    registers.  The stop is on the true residual (FP64 row sums), so in FP64 it holds up to the
+    rounding of the squared norms: 1e-5 (1 + 1e-4)."""
+    import scipy.sparse as sp
+    rp, ci, vals, b = _band(n, reach)
+    status, x, iters, rel, launches = _noalloc_launches(rp, ci, vals, b)
+    assert launches >= 1
     A = sp.bsr_matrix((vals.astype(np.float64), ci, rp), shape=(3 * n, 3 * n))
     res = np.linalg.norm(b - A @ x.astype(np.float64)) / np.linalg.norm(b)
     print("%d rows, reach %d: status %d, %d iterations, residual %.3g, in FP64 %.3g" % (n, reach, status, iters, rel, res))
@@ -132,3 +148,17 @@ def test_noalloc_sizes_and_row_lengths(n, reach):
     if iters > 2:
         status, x, iters, rel = _noalloc(rp, ci, vals, b, maxit=2)
         assert status != CS_OK and iters == 2 and np.isfinite(x).all()
+
+
+def test_noalloc_launch_that_fails_is_repeated_separately():
+    """A refused launch, and a workgroup that gives up at any meeting of the 2 i of i iterations (its peers'
+    next wait runs out, 5 ms here; after the last there is none): the separate launches' result, bit for
+    bit that of the one launch."""
+    rp, ci, vals, b = _band(1000, 20)  # four workgroups, rows of more blocks than the registers hold
+    status, ref, iters, rel, launches = _noalloc_launches(rp, ci, vals, b)
+    assert status == CS_OK and launches == 1
+    for fault in [{"refuse": 1}] + [{"lose_wg": 1, "lose_at": at, "wait_s": 5e-3}
+                                    for at in (1, 2, 2 * iters - 1, 2 * iters, 2 * iters + 1)]:
+        s, x, i, r, launches = _noalloc_launches(rp, ci, vals, b, **fault)
+        assert launches == (1 if fault.get("lose_at") == 2 * iters + 1 else 0), fault
+        assert (s, i, r) == (status, iters, rel) and np.array_equal(x, ref), fault

@@ -6,8 +6,8 @@ import pytest
 
 from clothsimulator_amd import CS_MESH_CLOTH, Simulator, scenes
 from clothsimulator_amd._cabi import (CS_FLAG_FIXED_TUNING, CS_FLAG_INSTANCES, CS_FLAG_TIME_KERNELS, CS_PRECOND_AMG,
-                                      CS_PRECOND_AMG_LEARNED, CS_PRECOND_LEARNED, MeshArrays, default_params,
-                                      material_struct)
+                                      CS_PRECOND_AMG_LEARNED, CS_PRECOND_BLOCK_JACOBI, CS_PRECOND_LEARNED, MeshArrays,
+                                      default_params, material_struct)
 
 pytestmark = pytest.mark.gpu
 
@@ -108,7 +108,8 @@ def test_contacts_equal_launched():
     _compare(spec, x, np.zeros_like(x))
 
 
-def test_rows_wider_than_the_registers():
+@pytest.mark.parametrize("precond", [CS_PRECOND_BLOCK_JACOBI, CS_PRECOND_LEARNED])
+def test_rows_wider_than_the_registers(precond):
     """A fan of 40 triangles: its hub's row has 41 blocks, the rim's rows 6 or fewer."""
     k = 40
     a = 2 * np.pi * np.arange(k) / k
@@ -116,7 +117,7 @@ def test_rows_wider_than_the_registers():
     faces = np.array([[0, 1 + i, 1 + (i + 1) % k] for i in range(k)], np.int32)
     mesh = MeshArrays(np.column_stack([xy, np.zeros(k + 1)]), faces)
     spec = scenes.SceneSpec("fan", default_params(), [scenes.ClothSpec(mesh, material_struct())], [], 1)
-    _compare(spec, *_state(spec, amp=1e-3))
+    _compare(spec, *_state(spec, amp=1e-3), precond=precond)
 
 
 def test_columns_too_far_for_16_bits_are_solved_by_launches():
@@ -183,7 +184,7 @@ def _fault_case(case):
         spec.params.flags |= CS_FLAG_FIXED_TUNING
         return spec
     spec = scenes.crumple(33, height=0.01, sigma=0.05 / 33)
-    spec.params.precond = {"jacobi": 0, "learned": CS_PRECOND_LEARNED, "amg": CS_PRECOND_AMG}[case]
+    spec.params.precond = {"jacobi": CS_PRECOND_BLOCK_JACOBI, "learned": CS_PRECOND_LEARNED, "amg": CS_PRECOND_AMG}[case]
     return spec
 
 

@@ -28,6 +28,29 @@ struct StatusError : std::runtime_error {
 
 #define CS_LAUNCH_CHECK() CS_HIP(hipGetLastError())
 
+// Whether the next solve is attempted in one cooperative launch.  After a failed attempt the next `pause`
+// solves go straight to separate launches; failures in a row double the pause.  A refused launch costs
+// little and passes when the process that holds the device's cooperative queue is done with it; a wait that
+// ran out costs its bound (2 s), so its pauses are longer.
+struct OneLaunch {
+    int skip = 0, pause = 0;
+    bool attempt() {
+        if (skip == 0) return true;
+        skip--;
+        return false;
+    }
+    void worked() { pause = 0; }
+    void refused() { fail(1, 255); }
+    void ranOut() { fail(255, 65535); }
+
+private:
+    void fail(int least, int most) {
+        const int next = 2 * pause + 1;
+        pause = next < least ? least : next > most ? most : next;
+        skip = pause;
+    }
+};
+
 inline int cdiv(long a, long b) { return (int)((a + b - 1) / b); }
 
 // Grow-only device allocation.  Growing frees the old block (hipFree waits for

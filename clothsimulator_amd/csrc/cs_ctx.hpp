@@ -251,7 +251,7 @@ struct cs_ctx {
     cs::PcgScalars* hScal = nullptr;  // pinned
     // whole solves in one launch (cs_ppcg.hip): system table, block -> (system, workgroup) map, slots
     cs::DBuf ppTab, ppMap, ppSlots;
-    bool ppOff = false;  // refused a launch: solve with separate launches
+    cs::OneLaunch ppOnce;
     int ppLaunches = 0;  // launches that held the last solve, 0: separate ones
     cs_launch_fault ppFault{};  // (testing)
     // batched solve of independent cloths: per-cloth table, block -> cloth map, partials, scalars

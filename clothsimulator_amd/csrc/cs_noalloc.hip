@@ -12,8 +12,8 @@
 // race.
 //
 // The iterations run in one cooperative launch (k_na_loop), a row per thread, its first blocks in
-// registers; where that launch is refused, or a wait in it runs out, as separate launches with one
-// scalar record read back every NA_CHUNK iterations.  Both give the same bits.
+// registers; where that launch is refused, or a wait in it runs out, and for a while after (OneLaunch), as
+// separate launches with one scalar record read back every NA_CHUNK iterations.  Both give the same bits.
 #include <cfloat>
 #include <mutex>
 
@@ -491,21 +491,25 @@ __global__ void k_na_clear_slots(uint64_t* slots) {
     slots[blockIdx.x * NA_TB + threadIdx.x] = 0;
 }
 
-// The scratch address on each device, looked up once per device with that device current.
+// The scratch address on each device, looked up once per device with that device current, and whether the
+// device's next call attempts the one launch (both paths give the same bits).
 std::mutex gNaMutex;
-float* gNaBase[64] = {};
+struct NaDevice {
+    float* base = nullptr;
+    OneLaunch once;
+} gNaDevice[64];
 
-float* scratch_base() {
+NaDevice& current_device() {
     int dev = 0;
     CS_HIP(hipGetDevice(&dev));
     if (dev < 0 || dev >= 64) throw StatusError(CS_E_NO_DEVICE, "device index out of range");
     std::lock_guard<std::mutex> lock(gNaMutex);
-    if (!gNaBase[dev]) {
+    if (!gNaDevice[dev].base) {
         void* p = nullptr;
         CS_HIP(hipGetSymbolAddress(&p, HIP_SYMBOL(scratch)));
-        gNaBase[dev] = static_cast<float*>(p);
+        gNaDevice[dev].base = static_cast<float*>(p);
     }
-    return gNaBase[dev];
+    return gNaDevice[dev];
 }
 
 // The iterations in one launch.  False: refused (another process holds the device's cooperative
@@ -523,7 +527,12 @@ bool loop_at_once(hipStream_t s, int nb, int n, const int* rp, const int* ci, co
 
 int solve_noalloc(hipStream_t s, int n, const int* rp, const int* ci, const float* vals, const float* b, float* x,
                   float tol, int maxit, int* iters, float* relres, const cs_launch_fault& fault, int* launches) {
-    NaPtr P = carve(scratch_base());
+    NaDevice& dev = current_device();
+    auto locked = [&](auto&& f) {
+        std::lock_guard<std::mutex> lock(gNaMutex);
+        return f(dev.once);
+    };
+    NaPtr P = carve(dev.base);
     P.ticks = fault.wait_s > 0.0f ? (unsigned long long)(fault.wait_s * 1e8f) : NA_WAIT_TICKS;
     P.loseWg = fault.lose_wg;
     P.loseAt = fault.lose_at;
@@ -543,7 +552,7 @@ int solve_noalloc(hipStream_t s, int n, const int* rp, const int* ci, const floa
         CS_HIP(hipStreamSynchronize(s));
     };
     start();
-    bool once = true;
+    bool once = locked([](OneLaunch& o) { return o.attempt(); });
     int restart = 0;
     // The loop stops on its recursive residual; as in cs_solve, only the true residual (FP64 row
     // sums) accepts the result, otherwise the loop goes on from it, at most NA_RESTARTS times.
@@ -551,7 +560,9 @@ int solve_noalloc(hipStream_t s, int n, const int* rp, const int* ci, const floa
         if (once) {
             once = loop_at_once(s, nb, n, rp, ci, vals, x, P, fault.refuse != 0);
             read();
+            if (!once) locked([](OneLaunch& o) { o.refused(); });
             if (once && (!h.done || h.lost)) {  // a wait ran out: from the start
+                locked([](OneLaunch& o) { o.ranOut(); });
                 once = false;
                 restart = 0;
                 start();
@@ -579,6 +590,7 @@ int solve_noalloc(hipStream_t s, int n, const int* rp, const int* ci, const floa
         read();
         if (h.done || restart == NA_RESTARTS) break;
     }
+    if (once) locked([](OneLaunch& o) { o.worked(); });
     if (iters) *iters = h.iters;
     if (relres) *relres = h.bb > 0.0f ? sqrtf(h.rr / h.bb) : 0.0f;
     if (launches) *launches = once ? 1 + restart : 0;

@@ -20,8 +20,8 @@
 // sums and the continuations from it, as pcg_solve's.  The workgroups of a group wait for each
 // other, so they must all be resident: launches are cooperative and no larger than the device
 // holds at once.  One process at a time gets a device's cooperative queue: where the launch is
-// refused, and if a wait (each is bounded in time) runs out, the context solves with separate
-// launches from then on.
+// refused, and if a wait (each is bounded in time) runs out, the solve is made with separate launches, and
+// so are the context's next ones for a while (OneLaunch).
 //
 // The preconditioner is part of the kernel: block Jacobi in the update; the learned factor's two
 // sweeps; or the multigrid cycle with the rows of each coarse level spread over the group's waves, a
@@ -1084,7 +1084,7 @@ bool run_plan(cs_ctx* C, const Plan& p, const std::vector<int>& cloths, int pre,
             // too large, or another process holds the device's cooperative queue
             (void)hipGetLastError();
             CS_HIP(hipStreamSynchronize(s));
-            C->ppOff = true;
+            C->ppOnce.refused();
             return false;
         }
     }
@@ -1092,7 +1092,7 @@ bool run_plan(cs_ctx* C, const Plan& p, const std::vector<int>& cloths, int pre,
     CS_HIP(hipStreamSynchronize(s));
     for (int k = 0; k < n; k++)
         if (!h[k].done || h[k].lost) {
-            C->ppOff = true;
+            C->ppOnce.ranOut();
             return false;
         }
     for (int k = 0; k < n; k++) {
@@ -1106,7 +1106,7 @@ bool run_plan(cs_ctx* C, const Plan& p, const std::vector<int>& cloths, int pre,
 }
 
 bool allowed(const cs_ctx* C) {
-    return !C->ppOff && !(C->P.flags & (CS_FLAG_TIME_KERNELS | CS_FLAG_GRAPH_CYCLES));
+    return !(C->P.flags & (CS_FLAG_TIME_KERNELS | CS_FLAG_GRAPH_CYCLES));
 }
 
 }  // namespace
@@ -1118,7 +1118,9 @@ bool ppcg_solve(cs_ctx* C, int c, bool amg, bool learned, int* iters, float* rel
     const int pre = amg ? PRE_AMG : learned ? PRE_LEARNED : PRE_JACOBI;
     const std::vector<int> one{c};
     const Plan p = plan_for(C, one, pre, true);
-    return p.fits && run_plan(C, p, one, pre, true, iters, relres, converged);
+    if (!p.fits || !C->ppOnce.attempt() || !run_plan(C, p, one, pre, true, iters, relres, converged)) return false;
+    C->ppOnce.worked();
+    return true;
 }
 
 bool ppcg_solve_batch(cs_ctx* C, bool amg, int* iters, float* relres, int* converged) {
@@ -1133,6 +1135,7 @@ bool ppcg_solve_batch(cs_ctx* C, bool amg, int* iters, float* relres, int* conve
         plan[k] = plan_for(C, part[k], k ? PRE_AMG : PRE_JACOBI, false);
         if (!plan[k].fits) return false;
     }
+    if (!C->ppOnce.attempt()) return false;
     if (amg) bamg_prepare(C);
     for (int k = 0; k < 2; k++) {
         if (part[k].empty()) continue;
@@ -1149,6 +1152,7 @@ bool ppcg_solve_batch(cs_ctx* C, bool amg, int* iters, float* relres, int* conve
             converged[part[k][j]] = cv[j];
         }
     }
+    C->ppOnce.worked();
     return true;
 }
 

@@ -229,6 +229,31 @@ def test_a_workgroup_that_gives_up_falls_back(case, at):
     assert launches == 0 and it == rit and np.array_equal(dv, ref)
 
 
+@pytest.mark.parametrize("fault,pauses", [({"refuse": 1}, (1, 3)), ({"lose_wg": 1, "lose_at": 3, "wait_s": 2e-3}, (255,))])
+def test_one_launch_is_tried_again_after_a_pause(fault, pauses):
+    """A refusal passes: the solves after it take separate launches (1, then 3, ... while it is refused
+    again), then the launch is tried again.  A wait that ran out pauses it for 255 solves."""
+    sim = Simulator(scenes.hang(23))  # three workgroups
+    sim.assemble(0)
+
+    def launches():
+        sim.solve(0)
+        return sim.solve_launches()
+
+    assert launches() == 1
+    for n in pauses:
+        sim.set_launch_fault(**fault)
+        assert launches() == 0
+        if n == pauses[-1]:
+            sim.set_launch_fault()
+        assert [launches() for _ in range(n)] == [0] * n
+    assert [launches() for _ in range(3)] == [1] * 3
+    sim.set_launch_fault(refuse=1)  # a success ends the doubling
+    assert launches() == 0
+    sim.set_launch_fault()
+    assert [launches() for _ in range(2)] == [0, 1]
+
+
 def test_a_workgroup_that_gives_up_at_the_last_meeting_is_noticed():
     """At the last meeting no peer waits for the lost workgroup again, and the record is complete: only
     the lost workgroup's own word tells.  A block-Jacobi solve of i iterations meets 2 i + 3 times, and

@@ -153,7 +153,9 @@ def test_noalloc_sizes_and_row_lengths(n, reach):
 def test_noalloc_launch_that_fails_is_repeated_separately():
     """A refused launch, and a workgroup that gives up at any meeting of the 2 i of i iterations (its peers'
     next wait runs out, 5 ms here; after the last there is none): the separate launches' result, bit for
-    bit that of the one launch."""
+    bit that of the one launch.  The calls after it take separate launches too, one after a refusal and 255
+    after a wait that ran out, then the launch is tried again."""
+    small = _band(2, 1)
     rp, ci, vals, b = _band(1000, 20)  # four workgroups, rows of more blocks than the registers hold
     status, ref, iters, rel, launches = _noalloc_launches(rp, ci, vals, b)
     assert status == CS_OK and launches == 1
@@ -162,3 +164,6 @@ def test_noalloc_launch_that_fails_is_repeated_separately():
         s, x, i, r, launches = _noalloc_launches(rp, ci, vals, b, **fault)
         assert launches == (1 if fault.get("lose_at") == 2 * iters + 1 else 0), fault
         assert (s, i, r) == (status, iters, rel) and np.array_equal(x, ref), fault
+        pause = 0 if launches else 1 if "refuse" in fault else 255
+        assert all(_noalloc_launches(*small)[4] == 0 for _ in range(pause)), fault
+        assert _noalloc_launches(*small)[4] >= 1, fault

@@ -29,12 +29,17 @@ constexpr int NA_MAX = CS_NOALLOC_MAX_NODES;
 constexpr int NA_TB = 256;                    // threads per workgroup, one row each
 constexpr int NA_MAXB = NA_MAX / NA_TB;       // workgroups (partial-sum slots) at most
 constexpr int NA_CHUNK = 16;                  // iterations between host reads
+// Blocks of a row at most in the one launch (k_na_loop), which sends wider ones to the separate launches: they
+// walk a lone long row faster (a hub row of 200 blocks 3.6 ms a solve against 2.8 in one launch, of 1,000
+// blocks 11.1 against 12.6; 1,000 rows of 301 blocks 4.8 against 5.9).
+constexpr int NA_WIDE = 256;
 constexpr int NA_RESTARTS = 4;                // continuations from the true residual at most
 
 struct NaScal {
     float bb, rz, rr, alpha, beta, tol2bb;
     int done, iters, maxit, bad;
     int lost;  // a workgroup of k_na_loop gave up waiting: x is incomplete
+    int wide;  // a row has more than NA_WIDE blocks
 };
 
 // float offsets into the scratch array
@@ -110,6 +115,7 @@ __global__ void __launch_bounds__(NA_TB) k_na_init(int n, const int* __restrict_
     float bb = 0.0f, rz = 0.0f;
     if (i < n) {
         int diag = -1;
+        if (rp[i + 1] - rp[i] > NA_WIDE) P.sc->wide = 1;
         bool cols_ok = true;  // a column outside [0, n) would make the SpMV read outside the scratch vectors
         for (int k = rp[i]; k < rp[i + 1]; k++) {
             const int j = ci[k];
@@ -292,7 +298,10 @@ __global__ void k_na_clear(NaScal* sc) {
 // becomes visible; each thread forms its neighbours' d = z + beta d itself.
 // 8,100 rows of 13 blocks: a solve of 144 iterations 2.88 ms in separate launches, 1.44 here.
 constexpr int NA_RS = 14;                                      // blocks of a row in registers
+constexpr int NA_NT = 2;                                       // further blocks in flight together
 constexpr unsigned long long NA_WAIT_TICKS = 200000000ull;     // 2 s of the 100 MHz wall clock; a wait's bound
+
+typedef float f3u __attribute__((ext_vector_type(3), aligned(4)));
 
 __device__ __forceinline__ void put1(float* p, float v) {
     __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -373,7 +382,7 @@ __device__ bool na_meet(float (&v)[NS], int nb, unsigned ep, const NaPtr& P, uns
 __global__ void __launch_bounds__(NA_TB, 2) k_na_loop(int n, const int* __restrict__ rp, const int* __restrict__ ci,
                                                       const float* __restrict__ vals, float* __restrict__ x, NaPtr P) {
     __shared__ unsigned ranOut;
-    if (P.sc->done) return;
+    if (P.sc->done || P.sc->wide) return;
     if (threadIdx.x == 0) ranOut = P.loseWg == (int)blockIdx.x ? P.loseAt : 0;
     auto lost = [&]() {
         if (threadIdx.x == 0) P.sc->lost = 1;
@@ -441,10 +450,25 @@ __global__ void __launch_bounds__(NA_TB, 2) k_na_loop(int n, const int* __restri
 #pragma unroll
             for (int u = 0; u < 7; u++) add(a[g + u], w[u]);
         }
-        for (int k = k0 + NA_RS; k < k1; k++) {
-            float w[3];
-            dir(ci[k], w);
-            add(vals + (size_t)k * 9, w);
+        // further blocks, NA_NT in flight together, a row's vector in one load: bound by the loads a lone lane
+        // issues (30,000 rows of 101 blocks: 25.6 ms in separate launches, 29.0 here with scalar loads one block
+        // at a time, 20.7 now), which the blocks in registers are not (there the wider loads spill and lose 10 %)
+        for (int k = k0 + NA_RS; k < k1; k += NA_NT) {
+            float A[NA_NT][9], w[NA_NT][3];
+#pragma unroll
+            for (int u = 0; u < NA_NT; u++) {
+                const int kk = min(k + u, k1 - 1), j = ci[kk];
+#pragma unroll
+                for (int c = 0; c < 9; c++) A[u][c] = vals[(size_t)kk * 9 + c];
+                const f3u zj = *(const f3u*)(P.z + 3 * j);
+                f3u dj = zj;
+                if (it != first) dj = *(const f3u*)(dp + 3 * j);
+#pragma unroll
+                for (int c = 0; c < 3; c++) w[u][c] = it == first ? zj[c] : zj[c] + beta * dj[c];
+            }
+#pragma unroll
+            for (int u = 0; u < NA_NT; u++)
+                if (k + u < k1) add(A[u], w[u]);
         }
         float v1[1] = {0.0f};
         if (live)
@@ -560,12 +584,16 @@ int solve_noalloc(hipStream_t s, int n, const int* rp, const int* ci, const floa
         if (once) {
             once = loop_at_once(s, nb, n, rp, ci, vals, x, P, fault.refuse != 0);
             read();
-            if (!once) locked([](OneLaunch& o) { o.refused(); });
-            if (once && (!h.done || h.lost)) {  // a wait ran out: from the start
+            if (!once) {
+                locked([](OneLaunch& o) { o.refused(); });
+            } else if (h.lost || !(h.done || h.wide)) {  // a wait ran out: from the start
                 locked([](OneLaunch& o) { o.ranOut(); });
                 once = false;
                 restart = 0;
                 start();
+            } else {
+                locked([](OneLaunch& o) { o.worked(); });
+                once = h.done;  // not done: rows too wide, the solve is as it was
             }
         }
         if (!once)
@@ -590,7 +618,6 @@ int solve_noalloc(hipStream_t s, int n, const int* rp, const int* ci, const floa
         read();
         if (h.done || restart == NA_RESTARTS) break;
     }
-    if (once) locked([](OneLaunch& o) { o.worked(); });
     if (iters) *iters = h.iters;
     if (relres) *relres = h.bb > 0.0f ? sqrtf(h.rr / h.bb) : 0.0f;
     if (launches) *launches = once ? 1 + restart : 0;

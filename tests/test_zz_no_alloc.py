@@ -167,3 +167,24 @@ def test_noalloc_launch_that_fails_is_repeated_separately():
         pause = 0 if launches else 1 if "refuse" in fault else 255
         assert all(_noalloc_launches(*small)[4] == 0 for _ in range(pause)), fault
         assert _noalloc_launches(*small)[4] >= 1, fault
+
+
+@pytest.mark.parametrize("n,launched", [(256, False), (257, True)])
+def test_noalloc_rows_too_wide_for_one_launch(n, launched):
+    """One row and column full (n blocks in row 0): up to 256 blocks in one launch, more in separate ones;
+    the same bits either way."""
+    rng = np.random.default_rng(n)
+    rows = [sorted({0, i} | ({i - 1} if i > 1 else set()) | ({i + 1} if 0 < i < n - 1 else set())) for i in range(n)]
+    rows[0] = list(range(n))
+    rp = np.concatenate([[0], np.cumsum([len(r) for r in rows])]).astype(np.int32)
+    ci = np.concatenate(rows).astype(np.int32)
+    diag = ci == np.repeat(np.arange(n), np.diff(rp))
+    # couplings of -0.02: row 0's sum to 0.02 n < 16, the others' to 0.06 < 4 (positive definite)
+    vals = np.where(diag[:, None], 4.0, -0.02) * np.eye(3).reshape(1, 9)
+    vals[0] *= 4.0
+    b = rng.standard_normal(3 * n).astype(np.float32)
+    status, x, iters, rel, launches = _noalloc_launches(rp, ci, vals.astype(np.float32), b)
+    assert status == CS_OK and (launches == 0) == launched
+    other = _noalloc_launches(rp, ci, vals.astype(np.float32), b, refuse=1)
+    assert other[4] == 0 and other[0] == status and other[2:4] == (iters, rel) and np.array_equal(other[1], x)
+    assert _noalloc_launches(*_band(2, 1))[4] == 0 and _noalloc_launches(*_band(2, 1))[4] >= 1  # the pause after it

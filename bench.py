@@ -24,9 +24,10 @@ the whole preconditioner (M^-1 = G^T G), and with the multigrid cycle smoothed
 by block Jacobi, each on a fresh context.
 
 Prints one JSON line: node-steps/s and CG iterations per step of the measured
-run, the same for the comparison runs, the roofline of the dominant kernel (the
-PCG SpMV, timed live with HIP events on the library's stream) and a CPU
-baseline (the oracle restatement on the host cores, on a bounded sample: the
+run, the same for the comparison runs, the roofline of the PCG SpMV (timed with
+HIP events on the library's stream, in a further run of the same steps: the
+sampling keeps solves that fit one launch in separate ones, which the measured
+runs do not) and a CPU baseline (the oracle restatement on the host cores, on a bounded sample: the
 first step of the same workload).
 """
 import argparse
@@ -186,6 +187,7 @@ def run(workload, precond, steps, warmup, timed, extra_flags=0):
     span = max(steps, spec.steps)
     sel = set(timed_steps(steps, span))
     iters, contacts, failed, failures = [], [], 0, []
+    one_launch = 0
     elapsed = 0.0
     t_all = time.perf_counter()
     for k in range(span):
@@ -204,11 +206,12 @@ def run(workload, precond, steps, warmup, timed, extra_flags=0):
                     precond, k, s, st.pcg_converged, st.pcg_rel_residual), file=sys.stderr, flush=True)
             iters.append(st.pcg_iters)
             contacts.append(st.n_contact_blocks)
+            one_launch += sim.solve_launches() > 0
         if (k + 1) % 50 == 0:
             print("%s step %d/%d  %.1f s  cg %d" % (precond, k + 1, span, time.perf_counter() - t_all, st.pcg_iters),
                   file=sys.stderr, flush=True)
     out = {"spec": spec, "elapsed": elapsed, "iters": iters, "contacts": contacts, "failed": failed,
-           "failures": failures,
+           "failures": failures, "one_launch": one_launch,
            "value": spec.n_cloth_nodes * len(sel) / elapsed, "ms_per_step": 1e3 * elapsed / len(sel),
            "span": span, "timed": len(sel)}
     if timed:
@@ -251,7 +254,8 @@ def sequential_sample(spec, precond, steps, k, batched_value):
 
 def summary(r):
     return {"value": r["value"], "ms_per_step": r["ms_per_step"], "cg_iters_mean": float(np.mean(r["iters"])),
-            "cg_iters_max": int(np.max(r["iters"])), "failed_steps": r["failed"], "failures": r["failures"]}
+            "cg_iters_max": int(np.max(r["iters"])), "failed_steps": r["failed"], "failures": r["failures"],
+            "steps_solved_in_one_launch": r["one_launch"]}
 
 
 def remesh_run(workload, frames, steps_per_frame=8):
@@ -336,24 +340,25 @@ def main():
     from clothsimulator_amd import scenes
 
     steps = a.steps if a.steps is not None else scenes.by_name(a.workload).steps
-    main_run = run(a.workload, a.precond, steps, a.warmup, True)
+    main_run = run(a.workload, a.precond, steps, a.warmup, False)
     spec = main_run["spec"]
     others = {}
     for p in [q for q in a.compare.split(",") if q and q != a.precond]:
         others[p] = run(a.workload, p, steps, a.warmup, False)
+    sampled = run(a.workload, a.precond, steps, a.warmup, True)
 
     n_nodes = spec.n_cloth_nodes
     c0 = spec.cloths[0]
     nnzb = sum(static_nnzb(c.mesh.faces, c.mesh.n_nodes) for c in spec.cloths)
-    nnzb_dyn = nnzb + float(np.mean(main_run["contacts"]))
+    nnzb_dyn = nnzb + float(np.mean(sampled["contacts"]))
     # algorithmic bytes of one SpMV launch: 36 B values + 4 B column index per block; per node
     # z and the previous direction read once (16 B each), the new direction (16 B) and q (12 B)
     # written once
     bytes_per_launch = 40.0 * nnzb_dyn + 60.0 * n_nodes
     # every sampled SpMV is bracketed by an event pair; an empty pair recorded just before it
     # measures the markers' own latency, which is subtracted
-    spmv_ms, spmv_n = main_run["spmv"]
-    pair_ms, pair_n = main_run["pair"]
+    spmv_ms, spmv_n = sampled["spmv"]
+    pair_ms, pair_n = sampled["pair"]
     marker_s = (pair_ms / pair_n) * 1e-3 if pair_n else 0.0
     avg_s = (spmv_ms / spmv_n) * 1e-3 - marker_s if spmv_n else float("nan")
     achieved = bytes_per_launch / avg_s / 1e9 if spmv_n else None
@@ -394,6 +399,7 @@ def main():
             summary(others["jacobi"])["cg_iters_mean"] if "jacobi" in others else None),
         "failed_steps": ms["failed_steps"],
         "failures": ms["failures"],
+        "steps_solved_in_one_launch": ms["steps_solved_in_one_launch"],
         "roofline": roofline,
     }
     for p, r in others.items():

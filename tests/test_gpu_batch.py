@@ -41,17 +41,20 @@ def test_batched_instances_match_separate_runs():
     assert abs(its_batch - its_single) <= max(4, 0.02 * its_single), (its_batch, its_single)
 
 
-def test_batched_contacts_match_separate_runs():
+# in one launch; launched with 256 rows a workgroup
+@pytest.mark.parametrize("flags", [CS_FLAG_FIXED_TUNING, CS_FLAG_FIXED_TUNING | CS_FLAG_TIME_KERNELS])
+def test_batched_contacts_match_separate_runs(flags):
     """Instances resting on their spheres: the batched contact assembly (one sort over every
     cloth's blocks) gives each cloth the contact blocks of its own run."""
     spec = scenes.instances(count=3, seed=5, side_lo=17, side_hi=25, gap=0.004)
-    spec.params.flags |= CS_FLAG_FIXED_TUNING
+    spec.params.flags |= flags
     batch = Simulator(spec)
     contacts_batch = 0
     for _ in range(12):
         s, st = batch.step()
         assert s == 0, s
         contacts_batch += st.n_contact_blocks
+        assert batch.solve_launches() == (0 if flags & CS_FLAG_TIME_KERNELS else 1)
     assert contacts_batch > 0
     contacts_single = 0
     for k in range(3):
@@ -68,6 +71,30 @@ def test_batched_contacts_match_separate_runs():
     assert contacts_batch == contacts_single, (contacts_batch, contacts_single)
 
 
+def test_tuned_batched_contacts_match_separate_steps():
+    """The launched solve's first eight solves, every candidate shape twice.  128 rows a workgroup group the
+    partial sums differently from a separate run, so runs drift apart with the steps: each separate run
+    restarts every step from the batch's state, and every step must agree within 1e-5 m."""
+    spec = scenes.instances(count=3, seed=5, side_lo=17, side_hi=25, gap=0.004)
+    spec.params.flags |= CS_FLAG_TIME_KERNELS
+    batch = Simulator(spec)
+    sims = [Simulator(single(spec, k)) for k in range(3)]
+    contacts, worst = 0, 0.0
+    for step in range(12):
+        state = [batch.state(CS_MESH_CLOTH, k) for k in range(3)]
+        s, st = batch.step()
+        assert s == 0 and batch.solve_launches() == 0
+        assert batch.batch_tuning()[2] == min(step + 1, 8)
+        contacts += st.n_contact_blocks
+        for k, sim in enumerate(sims):
+            sim.set_state(CS_MESH_CLOTH, 0, *state[k])
+            s, st1 = sim.step()
+            assert s == 0
+            worst = max(worst, float(np.abs(batch.state(CS_MESH_CLOTH, k)[0] - sim.state()[0]).max()))
+    print("tuned batch: contact blocks %d, max|dx| per step %.3g" % (contacts, worst))
+    assert contacts > 0 and worst <= 1e-5
+
+
 @pytest.mark.parametrize("count,side_lo,side_hi,steps", [(3, 17, 25, 8), (256, 33, 65, 3)])
 def test_persistent_batched_solve_equals_launched(count, side_lo, side_hi, steps):
     """CS_FLAG_PERSISTENT_BATCH: the iterations between two polls as one cooperative launch with
@@ -76,16 +103,16 @@ def test_persistent_batched_solve_equals_launched(count, side_lo, side_hi, steps
     make about 2,500 (cloth, 256-row block) pairs, more than the roughly 1,500 workgroups the
     device holds at once, so each workgroup walks several; their static matrices (over 300 MB) also
     put the launched SpMV on non-temporal loads (above 128 MB), the persistent one on cached
-    ones."""
+    ones.  CS_FLAG_TIME_KERNELS keeps the small batch out of the one launch for the whole solve."""
     states = []
-    for flags in (CS_FLAG_PERSISTENT_BATCH, 0):
+    for flags in (CS_FLAG_TIME_KERNELS | CS_FLAG_PERSISTENT_BATCH, CS_FLAG_TIME_KERNELS):
         spec = scenes.instances(count=count, seed=5, side_lo=side_lo, side_hi=side_hi, gap=0.004)
         spec.params.flags |= CS_FLAG_FIXED_TUNING | flags
         sim = Simulator(spec)
         its = []
         for _ in range(steps):
             s, st = sim.step()
-            assert s == 0, s
+            assert s == 0 and sim.solve_launches() == 0, s
             its.append(st.pcg_iters)
         print("flags %d: iterations %s" % (flags, its), flush=True)
         states.append(([sim.state(CS_MESH_CLOTH, k) for k in range(count)], its))
@@ -152,9 +179,9 @@ def test_solves_in_one_launch_are_no_trials():
 
 
 def test_batch32_up_to_side129_matches_separate_runs_and_oracle():
-    """32 instances with sides drawn from 17..129 (most above 4,096 faces): the batch builds every
-    tree with the one-workgroup kernel, each separate run builds its large tree with the
-    per-mesh kernels.  The smallest and the largest instance, resynchronised with the oracle
+    """32 instances with sides drawn from 17..129 (most above 4,096 faces): the batch builds all its
+    trees with the grid-wide kernels, a separate run of an instance of at most 4,096 faces with the
+    one-workgroup kernel.  The smallest and the largest instance, resynchronised with the oracle
     before every step, are within 1e-5 m of the oracle's PCG step (1e-7 relative) after each of
     5 steps; then every instance, run 3 more steps alone from the batch's state, is within
     1e-5 m of the batch's own 3 steps."""

@@ -1,6 +1,7 @@
 """Independent instances with the multigrid preconditioner (CS_FLAG_INSTANCES + CS_PRECOND_AMG):
 every cloth keeps its own aggregation hierarchy, the batched PCG runs one V(1,1) cycle per cloth
-and iteration with each level launched once for all cloths.  The cycle is the single-cloth cycle
+and iteration, each level launched once for all cloths (CS_FLAG_TIME_KERNELS) or inside the one launch of
+the whole solves.  The cycle is the single-cloth cycle
 (same aggregates, Galerkin operators, smoother and exact coarsest solve); only the coarsest levels
 differ in form: the single-cloth solve applies its small levels as one dense operator, the batch
 runs them level by level.  So each instance must match its own single-cloth multigrid run to the
@@ -9,7 +10,8 @@ import numpy as np
 import pytest
 
 from clothsimulator_amd import CS_MESH_CLOTH, Simulator, scenes
-from clothsimulator_amd._cabi import CS_FLAG_FIXED_TUNING, CS_PRECOND_AMG, CS_PRECOND_BLOCK_JACOBI
+from clothsimulator_amd._cabi import (CS_FLAG_FIXED_TUNING, CS_FLAG_TIME_KERNELS, CS_PRECOND_AMG,
+                                      CS_PRECOND_BLOCK_JACOBI)
 
 pytestmark = pytest.mark.gpu
 
@@ -51,8 +53,10 @@ def _compare(spec, steps):
     return worst, np.array(its_b), its_s, worst_res
 
 
-def test_batched_multigrid_matches_separate_multigrid_runs():
+@pytest.mark.parametrize("flags", [0, CS_FLAG_TIME_KERNELS])
+def test_batched_multigrid_matches_separate_multigrid_runs(flags):
     spec = _batch(6, 3, 17, 65)
+    spec.params.flags |= flags
     worst, its_b, its_s, res = _compare(spec, 6)
     assert res <= 1e-5
     assert worst <= 1e-5
@@ -73,13 +77,15 @@ def test_streamed_batched_multigrid_matches_separate_runs():
     assert np.all(np.abs(its_b - its_s) <= np.maximum(3, 0.1 * its_s)), (its_b, its_s)
 
 
-def test_batched_multigrid_with_contacts_matches_separate_runs():
+@pytest.mark.parametrize("flags,launches", [(0, 1), (CS_FLAG_TIME_KERNELS, 0)])
+def test_batched_multigrid_with_contacts_matches_separate_runs(flags, launches):
     """Cloths resting on their spheres: level 1 of each cloth adds its own contact diagonal
     blocks (the batched contact assembly's per-cloth views).  In contact, a difference at the
     solve tolerance can change which impacts a later collision step finds, so a free run of
     12 steps drifts apart by more than one step's bar (3.2e-4 m measured): each separate run
     restarts every step from the batch's state, and every step must agree within 1e-5 m."""
     spec = _batch(4, 5, 17, 41, gap=0.004)
+    spec.params.flags |= flags
     batch = Simulator(spec)
     sims = [Simulator(single(spec, k)) for k in range(4)]
     worst, contacts, its_b, its_s = 0.0, 0, [], []
@@ -87,7 +93,7 @@ def test_batched_multigrid_with_contacts_matches_separate_runs():
         state = [batch.state(CS_MESH_CLOTH, k) for k in range(4)]
         s, st = batch.step()
         assert s == 0, s
-        assert st.pcg_rel_residual <= 1e-5
+        assert st.pcg_rel_residual <= 1e-5 and batch.solve_launches() == launches
         contacts += st.n_contact_blocks
         its_b.append(st.pcg_iters)
         n = 0
@@ -106,10 +112,12 @@ def test_batched_multigrid_with_contacts_matches_separate_runs():
     assert np.all(np.abs(its_b - its_s) <= np.maximum(3, 0.1 * its_s)), (its_b, its_s)
 
 
-def test_batch_mixes_multigrid_and_block_jacobi_cloths():
+@pytest.mark.parametrize("flags", [0, CS_FLAG_TIME_KERNELS])
+def test_batch_mixes_multigrid_and_block_jacobi_cloths(flags):
     """Cloths of 64 nodes or fewer (sides 5, 7 and 8 here) have no usable hierarchy: they run
     block Jacobi inside the same batched solve, as their single-cloth runs do."""
     spec = _batch(6, 3, 5, 33)
+    spec.params.flags |= flags
     sides = [int(round(np.sqrt(c.mesh.n_nodes))) for c in spec.cloths]
     print("sides", sides)
     assert sum(n <= 8 for n in sides) >= 2 and max(sides) >= 17

@@ -7,7 +7,7 @@ headline measurement, checked against the oracle and against FP64 arithmetic.
 * A contact state (the GPU's own run of 280 steps with the multigrid preconditioner: air drag
   holds the falling sheet near 1.2 m/s, so it lands on the ground plane after about 230 steps):
   candidate pairs and proximities bit-exact against
-  the oracle on the per-mesh trees, and, for every preconditioner, the solution of the assembled
+  the oracle on the grid-wide kernels' trees, and, for every preconditioner, the solution of the assembled
   system checked in FP64 on the host: ||b - A dv|| / ||b|| <= 1e-5 (the PCG stops on its
   recursive FP32 residual).
 * The learned preconditioner on this held-out system (its weights were trained on other

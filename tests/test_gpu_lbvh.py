@@ -1,12 +1,11 @@
 """GPU parity of the collision pipeline on meshes above 4,096 faces, and between separate cloths.
 
-A stage builds (and refits) a tree with the per-mesh kernels (Morton codes, multi-pass radix
-sort, Karras hierarchy, range tables, internal boxes) when the mesh has more than 32,768 faces,
-or more than 4,096 faces while the stage holds at most four such meshes; every smaller mesh is
-built by the one-workgroup batched kernel.  The drape, fold and crumple meshes here (49^2 to
-129^2 nodes: 4,608 to 32,768 faces, one such mesh per scene) therefore take the per-mesh path,
-the one the 129^2 and 513^2 workloads use; the five-cloth scene takes the batched path with the
-same mesh, and its pairs must be identical.
+A stage builds (and refits) all its trees with the grid-wide kernels (Morton codes, multi-pass radix
+sort, Karras hierarchy, range tables, internal boxes) when any mesh has more than 4,096 faces;
+otherwise the one-workgroup kernel builds each.  The drape, fold and crumple meshes here (49^2 to
+129^2 nodes: 4,608 to 32,768 faces) therefore take the grid-wide kernels, as the 129^2 and
+513^2 workloads do; a 45^2 cloth (3,872 faces) is built by the one-workgroup kernel on its own and by
+the grid-wide ones beside larger cloths, and its pairs must be identical.
 
 Bars: candidate pairs, proximity selection and impact lists bit-exact against the FP32 oracle
 (and pairs against brute force over every face pair); post-step positions within 1e-5 m of the
@@ -58,13 +57,13 @@ def _check_pairs(tag, sim, orc, cases, brute=True, refit=False):
         assert np.array_equal(_key(g), _key(o))
 
 
-def test_drape65_per_mesh_pairs_bitexact():
+def test_drape65_pairs_bitexact():
     spec, sim, orc, x, v = _lowered_drape(65)
     assert sim.counts(CS_MESH_CLOTH, 0)[1] == 8192
     _check_pairs("drape65", sim, orc, ((False, 2e-3), (True, 1e-4), (False, 5e-2)))
 
 
-def test_drape65_per_mesh_refit_bitexact():
+def test_drape65_refit_bitexact():
     """Trees built on one state and refit to another give the pairs a fresh build gives.  A refit
     keeps the build's leaf order, and a self pair is emitted with the face of lower sorted index
     as the query (src/BVHHelper.cu:167-168), so self pairs are compared unordered and their
@@ -103,31 +102,34 @@ def test_refit_without_trees_is_a_state_error():
         sim.lbvh_pairs(True, 1e-4, refit=True)  # trees built without the swept boxes
 
 
-def test_per_mesh_and_batched_trees_give_identical_pairs():
-    """One 65^2 cloth over its sphere (per-mesh trees) against the same cloth as cloth 0 of five
-    (five meshes above 4,096 faces: every tree from the batched kernel)."""
-    spec, sim, orc, x, v = _lowered_drape(65)
+def test_one_workgroup_and_grid_wide_trees_give_identical_pairs():
+    """One 45^2 cloth over its sphere (3,872 faces: the one-workgroup kernel) against the same cloth as
+    cloth 0 of three, the others of 65^2 nodes (8,192 faces: the grid-wide kernels for every tree)."""
+    spec, sim, orc, x, v = _lowered_drape(45)
     x = x.astype(np.float32)
     cloth = MeshArrays(x, spec.cloths[0].mesh.faces, uv=spec.cloths[0].mesh.uv,
                        face_verts=spec.cloths[0].mesh.face_verts)
-    far = [MeshArrays(x + np.array([5.0 * (k + 1), 0.0, 0.0], np.float32), cloth.faces, uv=cloth.uv,
-                      face_verts=cloth.face_verts) for k in range(4)]
-    spec5 = SceneSpec("five", spec.params, [ClothSpec(cloth, material_struct())] +
+    big = drape(65).cloths[0].mesh
+    far = [MeshArrays(big.x + np.array([5.0 * (k + 1), 0.0, 0.0], np.float32), big.faces, uv=big.uv,
+                      face_verts=big.face_verts) for k in range(2)]
+    spec3 = SceneSpec("three", spec.params, [ClothSpec(cloth, material_struct())] +
                       [ClothSpec(m, material_struct()) for m in far], spec.obstacles, 1)
-    sim5 = Simulator(spec5)
-    F = 8192
+    sim3 = Simulator(spec3)
+    F, G = cloth.n_faces, big.n_faces
+    assert F <= 4096 < G and spec.obstacles[0].n_faces <= 4096
     for ccd, th in ((False, 2e-3), (True, 1e-4), (False, 5e-2)):
-        a = sim.lbvh_pairs(ccd, th)
-        b = sim5.lbvh_pairs(ccd, th)
-        # cloth 0 and the sphere only: map the sphere's face ids (after 1 vs 5 cloths)
-        keep = (b < F).all(1) | ((b[:, 0] < F) & (b[:, 1] >= 5 * F))
-        b0 = b[keep].copy()
-        b0[b0 >= 5 * F] -= 4 * F
-        print("per-mesh %d, batched %d (cloth 0: %d)" % (len(a), len(b), len(b0)), flush=True)
-        assert len(a) > 0 and np.array_equal(_key(a), _key(b0))
-        # the far cloths see only themselves, and no pair crosses cloths
-        rest = b[~keep]
-        assert (rest[:, 0] // F == rest[:, 1] // F).all()
+        for refit in (False, True):
+            a = sim.lbvh_pairs(ccd, th, refit=refit)
+            b = sim3.lbvh_pairs(ccd, th, refit=refit)
+            # cloth 0 and the sphere only: map the sphere's face ids (after one or three cloths)
+            keep = (b[:, 0] < F) & ((b[:, 1] < F) | (b[:, 1] >= F + 2 * G))
+            b0 = b[keep].copy()
+            b0[b0 >= F + 2 * G] -= 2 * G
+            print("one workgroup %d, grid-wide %d (cloth 0: %d)" % (len(a), len(b), len(b0)), flush=True)
+            assert len(a) > 0 and np.array_equal(_key(a), _key(b0))
+            # the far cloths see only themselves, and no pair crosses cloths
+            rest = b[~keep] - F
+            assert (rest >= 0).all() and (rest[:, 0] // G == rest[:, 1] // G).all()
 
 
 def test_drape129_pairs_match_oracle():

@@ -318,6 +318,8 @@ def main():
     ap.add_argument("--cpu-direct", default="", metavar="WORKLOAD:STEPS,...",
                     help="also time the single-thread direct-solve CPU column on these windows "
                          "(e.g. drape129:20,crumple513:3); hang33 over its 100 steps always runs")
+    ap.add_argument("--no-roofline", action="store_true",
+                    help="leave out the further run that samples the SpMV (profiles of the measured runs alone)")
     ap.add_argument("--remesh-run", default="", metavar="WORKLOAD:FRAMES",
                     help="only run a remeshing workload (e.g. remesh_drape129:25: 8 steps then a remesh per frame) "
                          "and print its own JSON line")
@@ -345,32 +347,34 @@ def main():
     others = {}
     for p in [q for q in a.compare.split(",") if q and q != a.precond]:
         others[p] = run(a.workload, p, steps, a.warmup, False)
-    sampled = run(a.workload, a.precond, steps, a.warmup, True)
+    sampled = None if a.no_roofline else run(a.workload, a.precond, steps, a.warmup, True)
 
     n_nodes = spec.n_cloth_nodes
     c0 = spec.cloths[0]
     nnzb = sum(static_nnzb(c.mesh.faces, c.mesh.n_nodes) for c in spec.cloths)
-    nnzb_dyn = nnzb + float(np.mean(sampled["contacts"]))
-    # algorithmic bytes of one SpMV launch: 36 B values + 4 B column index per block; per node
-    # z and the previous direction read once (16 B each), the new direction (16 B) and q (12 B)
-    # written once
-    bytes_per_launch = 40.0 * nnzb_dyn + 60.0 * n_nodes
-    # every sampled SpMV is bracketed by an event pair; an empty pair recorded just before it
-    # measures the markers' own latency, which is subtracted
-    spmv_ms, spmv_n = sampled["spmv"]
-    pair_ms, pair_n = sampled["pair"]
-    marker_s = (pair_ms / pair_n) * 1e-3 if pair_n else 0.0
-    avg_s = (spmv_ms / spmv_n) * 1e-3 - marker_s if spmv_n else float("nan")
-    achieved = bytes_per_launch / avg_s / 1e9 if spmv_n else None
     from clothsimulator_amd._cabi import CS_FLAG_INSTANCES, CS_PRECOND_AMG, CS_PRECOND_BLOCK_JACOBI
     batched = bool(spec.params.flags & CS_FLAG_INSTANCES) and len(spec.cloths) > 1 \
         and spec.params.precond in (CS_PRECOND_BLOCK_JACOBI, CS_PRECOND_AMG)  # the batched solve of instances
-    roofline = {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
-                "frac": (achieved / HBM_PEAK_GBS) if achieved else None,
-                "traffic": read_traffic(a.workload, a.precond),
-                "kernel": "k_bpcg_spmv" if batched else "k_pcg_spmv",
-                "avg_us": avg_s * 1e6, "event_marker_us": marker_s * 1e6,
-                "launches_sampled": spmv_n, "bytes_per_launch": bytes_per_launch}
+    roofline = None
+    if sampled is not None:
+        nnzb_dyn = nnzb + float(np.mean(sampled["contacts"]))
+        # algorithmic bytes of one SpMV launch: 36 B values + 4 B column index per block; per node
+        # z and the previous direction read once (16 B each), the new direction (16 B) and q (12 B)
+        # written once
+        bytes_per_launch = 40.0 * nnzb_dyn + 60.0 * n_nodes
+        # every sampled SpMV is bracketed by an event pair; an empty pair recorded just before it
+        # measures the markers' own latency, which is subtracted
+        spmv_ms, spmv_n = sampled["spmv"]
+        pair_ms, pair_n = sampled["pair"]
+        marker_s = (pair_ms / pair_n) * 1e-3 if pair_n else 0.0
+        avg_s = (spmv_ms / spmv_n) * 1e-3 - marker_s if spmv_n else float("nan")
+        achieved = bytes_per_launch / avg_s / 1e9 if spmv_n else None
+        roofline = {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
+                    "frac": (achieved / HBM_PEAK_GBS) if achieved else None,
+                    "traffic": read_traffic(a.workload, a.precond),
+                    "kernel": "k_bpcg_spmv" if batched else "k_pcg_spmv",
+                    "avg_us": avg_s * 1e6, "event_marker_us": marker_s * 1e6,
+                    "launches_sampled": spmv_n, "bytes_per_launch": bytes_per_launch}
     ms = summary(main_run)
     out = {
         "metric": METRIC,

@@ -293,10 +293,11 @@ __global__ void k_na_clear(NaScal* sc) {
 }
 
 // ---- the iterations in one launch ------------------------------------------
-// Separate launches take 20 us an iteration, five of them (8,100 rows of 13 blocks), all latency.  Here
+// Separate launches take 20 us an iteration, five of them (8,100 rows of up to 11 blocks), all latency.  Here
 // an iteration is two meetings of the workgroups: for d.q, and for r.r and r.z, with which the new z
 // becomes visible; each thread forms its neighbours' d = z + beta d itself.
-// 8,100 rows of 13 blocks: a solve of 144 iterations 2.88 ms in separate launches, 1.44 here.
+// 8,100 rows of up to 11 blocks: a solve of 144 iterations 2.88 ms in separate launches, 1.44 here.  (One
+// register spills, 8 B of scratch a lane.)
 constexpr int NA_RS = 14;                                      // blocks of a row in registers
 constexpr int NA_NT = 2;                                       // further blocks in flight together
 constexpr unsigned long long NA_WAIT_TICKS = 200000000ull;     // 2 s of the 100 MHz wall clock; a wait's bound

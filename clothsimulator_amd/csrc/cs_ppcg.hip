@@ -27,12 +27,17 @@
 // sweeps; or the multigrid cycle with the rows of each coarse level spread over the group's waves, a
 // meeting per phase (restriction, pre-smoothing with residual, post-smoothing) instead of a launch.
 //
-// Measured (block Jacobi, solve time per iteration, separate launches -> here): 289 rows 14.1 -> 2.8 us,
-// 1,089 rows 13.5 -> 4.6, 16,641 rows with contacts 13.4 -> 7.5, 32,761 rows 13.9 -> 7.1,
-// 65,536 rows 18.0 -> 9.1, 129,600 rows 21.6 -> 15.3.
-// Solves with their set-up: learned factor 1,089 rows 3.9 -> 2.6 ms, 16,384 rows 9.0 -> 7.8, 32,400 rows
-// 9.5 -> 6.6; multigrid 289 rows 1.2 -> 0.8 ms, 4,225 rows 4.3 -> 3.7, 16,641 rows in contact 7.1 -> 5.4,
-// 32,400 rows 5.1 -> 3.6, 65,536 rows 7.4 -> 5.9.
+// Measured, solves with their set-up in ms (iterations), separate launches -> here:
+//   rows, regular grid   block Jacobi             learned factor          multigrid
+//   289                  1.08 -> 0.29 (81)        0.88 -> 0.57 (31)       0.96 -> 0.68 (19)
+//   1,089                1.39 -> 0.57 (104)       1.43 -> 0.90 (56)       0.94 -> 0.69 (24)
+//   16,641               4.32 -> 2.34 (318)       3.49 -> 2.55 (141)      2.38 -> 1.87 (39)
+//   65,536               7.90 -> 3.78 (400)       8.16 -> 5.73 (242)      3.96 -> 3.20 (48)
+//   131,044              23.4 -> 14.8 (1,074)     (launched)              (launched)
+//   rows, irregular mesh (17 to 20 blocks a row, those beyond the registers' 14 streamed)
+//   1,089                1.81 -> 0.82 (127)       1.99 -> 1.46 (69)       1.48 -> 1.07 (35)
+//   16,641               5.42 -> 3.13 (356)       6.17 -> 4.50 (190)      3.70 -> 2.67 (45)
+//   65,536               8.74 -> 4.65 (400)       10.8 -> 9.68 (270)      6.03 -> 5.05 (61)
 #include <algorithm>
 #include <cfloat>
 #include <cmath>
@@ -489,7 +494,8 @@ __global__ void __launch_bounds__(T, 2)  // 256 registers: the runtime refuses c
     // own holds up its wave, so the threads share the blocks evenly, CN in flight each and neighbours in
     // the matrix side by side, and a row's thread adds its products from LDS in order.  Solves, each row
     // walked by its thread -> shared: 129x129 drape block Jacobi 8.6 -> 7.9 ms, multigrid 5.7 -> 5.4;
-    // 201x201 fold learned 19.7 -> 17.6 (18.9 with 2,048 products of LDS); few contacts: the same.
+    // 201x201 fold learned, before its sweeps were grouped, 19.7 -> 17.6 (18.9 with 2,048 products of LDS);
+    // few contacts: the same.
     const int e0 = S.contacts ? S.cRowPtr[min(wg * T, nn)] : 0, e1 = S.contacts ? S.cRowPtr[min(wg * T + T, nn)] : 0;
     auto contacts = [&](auto& gat, auto&& add) {
         using W = decltype(gat(0));
@@ -930,7 +936,8 @@ int resident(cs_ctx* C, const void* f, int T) {
 }
 
 template <int PRE> const void* kernel_of(int T) {
-    constexpr int GR = PRE == PRE_LEARNED ? 4 : 7;  // without spilling
+    // (a further gather in flight spills; the learned kernel of 512 threads spills 7 registers with 4)
+    constexpr int GR = PRE == PRE_LEARNED ? 4 : 7;
     return T == 512 ? (const void*)k_ppcg<512, 14, 4, false, PRE> : (const void*)k_ppcg<256, 14, GR, false, PRE>;
 }
 const void* kernel_of(int T, bool local, int pre) {
@@ -969,19 +976,24 @@ Plan plan_for(cs_ctx* C, const std::vector<int>& cloths, int pre, bool dense) {
         local = local && S.nn <= 512;
         most = std::max(most, S.nn);
     }
-    // Large lone systems stream their factor or their coarse levels from memory either way (learned:
-    // 65,536 rows 11.0 against 13.6 ms a solve, 131,044 rows 23.8 against 20.0; multigrid: 90,000
-    // rows 7.8 against 8.7, 129,600 rows 10.4 against 9.8).
+    // Large lone systems stream their factor or their coarse levels from memory either way.  Multigrid: 97,969
+    // rows 4.16 ms a solve against 4.44 launched, 115,600 rows 4.81 against 4.63, 131,044 rows 5.00 against
+    // 4.75.  Learned: 65,536 rows 5.7 against 8.2; the line was drawn before its sweeps were grouped, and
+    // systems without contacts now gain beyond it too (90,000 rows 8.0 against 9.8, 131,044 rows 11.3 against
+    // 12.1); folded ones have not been measured there.
     if ((pre == PRE_LEARNED && most > 65536) || (pre == PRE_AMG && most > 98304)) return p;
     // more rows than the launches hold
     long rows = 0;
     for (int c : cloths) rows += 512l * cdiv(C->sys[c].nn, 512);
     const int launches = pre == PRE_JACOBI ? 2 : 1;
     if (rows > launches * 131072l) return p;
-    // Rows per workgroup: one workgroup and LDS for systems of 512 rows; otherwise a lone system is
-    // spread over more CUs by 256 (1,089 rows: 4.6 us an iteration with 256, 6.1 with 512), until the
-    // meeting of many workgroups costs more (65,536 rows: 12.6 us with 256, 9.1 with 512).  A batch
-    // fills the CUs anyway (32 cloths, 170,000 rows: 24.6 ms with 256, 15.9 with 512).
+    // Rows per workgroup: one workgroup and LDS for systems of 512 rows; otherwise a lone system is spread
+    // over more CUs by 256, until the meeting of many workgroups costs more.  Solves with 256 and 512, block
+    // Jacobi: 1,089 rows 0.57 and 0.68 ms, 8,281 rows 1.59 and 1.63, 16,641 rows 2.31 and 2.22, 24,336 rows
+    // 2.87 and 2.68, 28,900 rows 3.26 and 2.93, 65,536 rows 4.98 and 3.78; learned 24,336 rows 3.25 and 3.16,
+    // 28,900 rows 3.62 and 3.36; multigrid 2.37 and 2.16, 2.74 and 2.44: between 12,000 rows and the line the
+    // two are within 9 %.  A batch fills the CUs anyway (32 cloths, 170,000 rows: 24.6 ms with 256, 15.9
+    // with 512).
     const int T = p.T = local || n > 1 || most > 96 * 256 ? 512 : 256;
     p.f = kernel_of(T, local, pre);
     const int cap = resident(C, p.f, T);
